@@ -11,6 +11,7 @@
 #include <limits>
 #include <sstream>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <algorithm>
 #include <vector>
@@ -160,6 +161,21 @@ struct cf_crs {
 };
 
 namespace cf {
+BlockBudget* block_budget(int device) {
+    static std::mutex mu;
+    // never destroyed: handles may outlive static objects at process exit
+    static std::map<int, BlockBudget*>& all = *new std::map<int, BlockBudget*>();
+    std::lock_guard<std::mutex> lk(mu);
+    BlockBudget*& b = all[device];
+    if (!b) {
+        size_t free_b = 0, total_b = 0;
+        CF_HIP(hipMemGetInfo(&free_b, &total_b));  // of the current device, which the caller has set
+        b = new BlockBudget();
+        b->limit = total_b / 16;
+    }
+    return b;
+}
+
 // One-string diagonal parts and excitation lists (values included) of a
 // string table for the Hamiltonian H; the strings themselves do not depend on H.
 void fill_strtab(cf_ctx* ctx, const cf_ham* H, StrTab* t) {
@@ -309,6 +325,7 @@ bool make_sell(cf_crs* m, bool optional = false) {
     if (optional && m->scol.n != entries) {
         size_t free_b = 0, total_b = 0;
         CF_HIP(hipMemGetInfo(&free_b, &total_b));
+        free_b += block_budget(c->device)->held();  // kept blocks are given back when memory runs out
         if (entries * (12 + (m->want32 ? 4 : 0)) > free_b / 2) return false;
     }
     if (m->scol.n != entries) {
@@ -872,12 +889,8 @@ int cf_ctx_create(int device, cf_ctx** out) {
     std::unique_ptr<cf_ctx> c(new cf_ctx());
     c->device = device;
     CF_HIP(hipSetDevice(device));
-    // keep freed blocks in the device's stream-ordered pool for reuse
-    hipMemPool_t mp = nullptr;
-    CF_HIP(hipDeviceGetDefaultMemPool(&mp, device));
-    uint64_t keep = UINT64_MAX;
-    CF_HIP(hipMemPoolSetAttribute(mp, hipMemPoolAttrReleaseThreshold, &keep));
     CF_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    c->blocks = std::make_shared<DeviceBlocks>(c->stream, block_budget(device));
     c->use();
     CF_HIP(hipHostMalloc((void**)&c->pinned, cf_ctx::kPinned * sizeof(double), hipHostMallocDefault));
     std::vector<uint64_t> hb((kMaxL + 1) * kBinomCols, 0);

@@ -21,7 +21,7 @@ using cf::ERR_HIP;
 using cf::SigmaArgs;
 using cf::SigmaShape;
 using cf::str_t;
-using cf::tls_alloc_stream;
+using cf::tls_blocks;
 using cf::HamDev;
 using cf::Exc;
 
@@ -34,6 +34,7 @@ struct TimerFamily {
 struct cf_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
+    std::shared_ptr<cf::DeviceBlocks> blocks;  // device memory of this stream, kept for reuse
     DBuf<uint64_t> binom;  // C(k, m): (kMaxL+1) x kBinomCols
     bool timing = false;
     std::map<std::string, TimerFamily> timers;
@@ -85,7 +86,7 @@ struct cf_ctx {
 
     void use() {
         CF_HIP(hipSetDevice(device));
-        tls_alloc_stream = stream;
+        tls_blocks = blocks;
     }
     hipEvent_t event() {
         if (!pool.empty()) {
@@ -118,18 +119,19 @@ struct cf_ctx {
         for (auto e : pool) (void)hipEventDestroy(e);
         if (pinned) (void)hipHostFree(pinned);
         if (blas_) (void)rocblas_destroy_handle(blas_);
-        // buffers ordered on the stream go back to the pool before it is destroyed
+        // the stream's blocks go back before it is destroyed
         binom.release();
         hx.release();
         hy.release();
         doci_tabs.clear();
         doci_blk.clear();
         if (bpinned) (void)hipHostFree(bpinned);
+        if (blocks) blocks->cache.close();
+        if (tls_blocks == blocks) tls_blocks.reset();
         if (stream) {
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
         }
-        if (tls_alloc_stream == stream) tls_alloc_stream = nullptr;
     }
 };
 
@@ -190,6 +192,8 @@ struct cf_sigma {
 };
 
 namespace cf {
+// The device's block caches and what they may keep together (1/16 of its memory).
+BlockBudget* block_budget(int device);
 // One-string diagonal parts and excitation lists of a string table for H.
 void fill_strtab(cf_ctx* ctx, const cf_ham* H, StrTab* t);
 // Diagonal of the space for its current Hamiltonian.

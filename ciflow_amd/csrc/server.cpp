@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "../../include/ciflow_amd.h"
+#include "capi_types.h"
 #include "common.h"
 #include "davbatch.h"
 #include "kernels.h"
@@ -441,6 +442,7 @@ int cf_server_create(int device, int slots, double hbm_budget_bytes, cf_server**
         size_t fr = 0, tot = 0;
         CF_HIP(hipSetDevice(device));
         CF_HIP(hipMemGetInfo(&fr, &tot));
+        fr += cf::block_budget(device)->held();  // kept blocks are given back when memory runs out
         S->budget = (uint64_t)(0.8 * (double)fr);
     } else {
         S->budget = (uint64_t)hbm_budget_bytes;
