@@ -1,31 +1,39 @@
-// Many small DOCI ground-state solves in one launch: the served stream's
-// small requests (DOCI spaces of up to 13,312 determinants, L <= 16 at half
+// Many small DOCI ground-state solves at once: the served stream's small
+// requests (DOCI spaces of up to 13,312 determinants, L <= 16 at half
 // filling), which the reference solves one after another
 // (OrbitalOptimization::update_cim -> set_ham -> build_ci -> solve,
-// SimulatedAnnealing.cpp:83-87, CIMethod.cpp:117-126,241-268).  Solved one
-// request at a time they are bound by their chain of about 600 short kernel
-// launches, not by arithmetic; here one workgroup runs a whole solve on one
-// CU and a launch carries every request of a batch, of any mix of sizes.
+// SimulatedAnnealing.cpp:83-87, CIMethod.cpp:117-126,241-268).
 //
-// Per workgroup: the DOCI matrix of DOCI::construct_CI_matrix
-// (CIMethod.cpp:611-660) applied without storing it -- the diagonal
-// 2 sum h_ii + sum_i (ii|ii) + sum_{k != l} (2 (kk|ll) - (kl|lk)) per row once,
-// and the pair hops j -> k with element V(j,j,k,k) from an L x L table in LDS
-// and target ranks from the position-major hop columns shared by every
-// request of the same (L, pairs) shape -- and plain FP64 Lanczos on it: the
-// Krylov vector v_j in LDS (the gathers of the product read it there), w,
-// v_{j-1} and the diagonal in the request's global scratch (rows tid + k NT,
-// each touched by one thread only), alpha_j and beta_j in LDS.  Every
-// `check` steps wave 0 finds the two lowest eigenvalues of the tridiagonal
-// T_m by Sturm-count multisection (64 lanes, one candidate each) and the
-// last components of their eigenvectors by inverse iteration, and applies
-// the solver's stopping tests: ||r_0|| = |beta_m z_m| <= tol |theta_0|, or the
-// Kato-Temple estimate ||r_0||^2 / (theta_1 - ||r_1|| - theta_0) <= tol_energy.
-// Without reorthogonalisation converged Ritz values reappear as copies; a
-// second value within 1e-10 |theta_0| of the first is such a copy and the
-// gap is taken to the next distinct one.  All reductions have a fixed order,
-// so a request's result does not depend on the rest of its batch.
+// The DOCI matrix of DOCI::construct_CI_matrix (CIMethod.cpp:611-660) is
+// applied without storing it -- the diagonal 2 sum h_ii + sum_i (ii|ii) +
+// sum_{k != l} (2 (kk|ll) - (kl|lk)) per row once, and the pair hops j -> k with
+// element V(j,j,k,k) -- in plain FP64 Lanczos, and every request of the batch
+// takes its step j in one launch:
+//   * a request's rows are split over `nchunk` workgroups.  Each of them reads
+//     the whole of H v_{j-1}, v_{j-1} and v_{j-2} (a few times n doubles from
+//     L2), forms alpha_{j-1}, the next vector and its norm itself, so that no
+//     workgroup waits for another, holds v_j in LDS and applies H to its own
+//     rows.  The sums run over a fixed thread mapping of all n rows, so a
+//     request's result depends neither on the split nor on the batch.
+//   * one more workgroup per request tests T_{j-1} for convergence meanwhile:
+//     one wave finds the lowest eigenvalue and another the second by
+//     Sturm-count multisection, each then the last component of its
+//     eigenvector, and the solver's stopping tests are ||r_0|| = |beta_m z_m|
+//     <= tol |theta_0|, or the Kato-Temple estimate ||r_0||^2 / (theta_1 -
+//     ||r_1|| - theta_0) <= tol_energy.  Without reorthogonalisation converged
+//     Ritz values reappear as copies; a second value within 1e-10 |theta_0| of
+//     the first is such a copy and the gap is taken to the next distinct one.
+// The host stays eight steps ahead and stops when the last request is done.
+//
+// What bounds it: a step is the latency of one launch, two reductions over n
+// and np nv dependent-free gathers a row.  One workgroup per request, with the
+// test on one of its waves, left most CUs idle and waited for a column from L2
+// at every hop: 48 requests of L=14 (3,432 rows) took 9.1 ms on 48 of 256 CUs;
+// now a step is 13 us, a step with a test 20-30 us, and the batch 1.7 ms (a
+// whole call 10.9 -> 3.1 ms, the rest of it the integrals' way to the GPU).
 #include "batch.h"
+
+#include <algorithm>
 
 namespace cf {
 
@@ -39,72 +47,107 @@ __device__ __forceinline__ double wave_sum64(double v) {
     return v;
 }
 
-// Sturm count: eigenvalues of T_m below x (LDL^T pivots of T - x I).
-__device__ int sturm_count(const double* al, const double* be, int m, double x) {
-    int c = 0;
-    double q = al[0] - x;
-    if (q < 0.0) ++c;
-    for (int i = 1; i < m; ++i) {
-        if (q == 0.0) q = 1e-300;
-        q = (al[i] - x) - be[i - 1] * be[i - 1] / q;
-        if (q < 0.0) ++c;
+// T_m of one convergence test, scaled to [-1, 1] by its Gershgorin bounds and
+// padded to whole blocks of kBlk elements, which are read from LDS together.
+// Signs are compared as sign bits: as conditions they went through the scalar
+// unit, and an element of a test cost 0.65 us instead of 0.1.
+constexpr int kBlk = 16;
+constexpr int kPadSteps = (kMaxSteps + kBlk - 1) / kBlk * kBlk;
+struct alignas(16) TestMatrix {
+    double a[kPadSteps];   // diagonal (padding 4: no sign change)
+    double b2[kPadSteps];  // b_{i-1}^2, the square of the element before
+    // from the last row to the first (element q is row i = m - 1 - q)
+    double ra[kPadSteps];  // diagonal
+    double rn[kPadSteps];  // b_i
+    double rb[kPadSteps];  // 1 / b_{i-1} (0 at row 0 and in the padding)
+};
+
+// Eigenvalues of T_m below x: sign changes of the leading minors p_0 .. p_m,
+// p_i = (a_i - x) p_{i-1} - b_{i-1}^2 p_{i-2} (one dependent FMA an element; a
+// zero counts as positive, its successor has the sign opposite to its
+// predecessor's, so the changes add up).
+__device__ __forceinline__ int sturm_count(const TestMatrix& T, int m, double x) {
+    int c = 0, sign = 0;
+    double pp = 0.0, p = 1.0;
+    for (int i0 = 0; i0 < m; i0 += kBlk) {
+        double a[kBlk], b2[kBlk];
+#pragma unroll
+        for (int q = 0; q < kBlk; ++q) {
+            a[q] = T.a[i0 + q] - x;
+            b2[q] = T.b2[i0 + q];
+        }
+#pragma unroll
+        for (int q = 0; q < kBlk; ++q) {
+            const double pn = fma(a[q], p, -(b2[q] * pp));
+            pp = p;
+            p = pn;
+            const int sg = __double2hiint(pn);
+            c += (int)((unsigned)(sg ^ sign) >> 31);
+            sign = sg;
+        }
+        const double big = fmax(fabs(p), fabs(pp));  // a block multiplies by 5^16 at most
+        const double sc = big > 1e100 ? 1e-100 : big < 1e-100 ? 1e100 : 1.0;
+        p *= sc;
+        pp *= sc;
     }
     return c;
 }
 
 // k-th smallest eigenvalue (k = 0, 1, ...) of T_m by multisection over one
 // wave: every lane tests one point, the bracket shrinks 65-fold per round.
-__device__ double kth_eigenvalue(const double* al, const double* be, int m, int k, double lo, double hi) {
+// `prev`: that eigenvalue of an earlier T (any value above 1: none).  It is an
+// upper bound (interlacing), and the first round's points lie at distances
+// below it that grow 1.75-fold from lane to lane, so near convergence four
+// rounds are saved.  The tests take the value to 1e-13, which the last
+// component and the gap need; a result is refined to 1e-16.
+__device__ double kth_eigenvalue(const TestMatrix& T, int m, int k, double prev, double width) {
     const int lane = threadIdx.x & 63;
-    for (int round = 0; round < 12; ++round) {
-        const double x = lo + (hi - lo) * (double)(lane + 1) / 65.0;
-        const int c = sturm_count(al, be, m, x);
+    double lo = -1.0, hi = 1.0;
+    const bool warm = prev < 1.0;
+    for (int round = 0; round < 13 && hi - lo > width; ++round) {
+        const bool w = warm && round == 0;
+        const double x = w ? prev - exp2(1.0 - 51.0 * (double)lane / 63.0) : lo + (hi - lo) * (double)(lane + 1) / 65.0;
         // the first lane whose point has more than k eigenvalues below it
-        const unsigned long long ball = __ballot(c > k);
+        const unsigned long long ball = __ballot(sturm_count(T, m, x) > k);
         const int first = ball ? __builtin_ctzll(ball) : 64;
-        const double nlo = lo + (hi - lo) * (double)first / 65.0;
-        const double nhi = first < 64 ? lo + (hi - lo) * (double)(first + 1) / 65.0 : hi;
-        if (nhi - nlo <= 1e-16 * fmax(1.0, fabs(nlo))) {
-            lo = nlo;
-            hi = nhi;
-            break;
-        }
-        lo = nlo;
+        const double nlo = first > 0 ? __shfl(x, first - 1, 64) : lo;
+        const double nhi = first < 64 ? __shfl(x, first < 64 ? first : 63, 64) : w ? fmin(1.0, prev + 2e-13) : hi;
+        lo = fmax(lo, nlo);
         hi = nhi;
     }
     return 0.5 * (lo + hi);
 }
 
-// Last component of the normalised eigenvector of T_m for eigenvalue theta:
-// two steps of inverse iteration (tridiagonal elimination), one thread.
-__device__ double last_component(const double* al, const double* be, int m, double theta, double* wk) {
-    double* d = wk;        // pivots
-    double* z = wk + kMaxSteps;
-    for (int i = 0; i < m; ++i) z[i] = 1.0;
-    for (int it = 0; it < 2; ++it) {
-        // forward elimination of (T - theta I) z_new = z
-        d[0] = al[0] - theta;
-        if (fabs(d[0]) < 1e-150) d[0] = 1e-150;
-        for (int i = 1; i < m; ++i) {
-            const double l = be[i - 1] / d[i - 1];
-            d[i] = (al[i] - theta) - l * be[i - 1];
-            if (fabs(d[i]) < 1e-150) d[i] = 1e-150;
-            z[i] -= l * z[i - 1];
+// |last component| of the normalised eigenvector of T_m for eigenvalue x by
+// the recurrence from its end, z_{i-1} = -((a_i - x) z_i + b_i z_{i+1}) /
+// b_{i-1}: the component is small and the others grow from it, which is the
+// stable direction; only a few digits are needed.
+__device__ __forceinline__ double last_component(const TestMatrix& T, int m, double x) {
+    double zn = 0.0, z = 1.0, last = 1.0, nrm = 1.0;
+    for (int i0 = 0; i0 < m; i0 += kBlk) {
+        double a[kBlk], b[kBlk], rb[kBlk];
+#pragma unroll
+        for (int q = 0; q < kBlk; ++q) {
+            a[q] = T.ra[i0 + q] - x;
+            b[q] = T.rn[i0 + q];
+            rb[q] = T.rb[i0 + q];
         }
-        z[m - 1] /= d[m - 1];
-        for (int i = m - 2; i >= 0; --i) z[i] = (z[i] - be[i] * z[i + 1]) / d[i];
-        double zmax = 0.0;  // scale first: the solve is near-singular by design
-        for (int i = 0; i < m; ++i) zmax = fmax(zmax, fabs(z[i]));
-        if (!(zmax > 0.0) || !(zmax < 1e300)) return 0.0;
-        double nrm = 0.0;
-        for (int i = 0; i < m; ++i) {
-            z[i] /= zmax;
-            nrm += z[i] * z[i];
+#pragma unroll
+        for (int q = 0; q < kBlk; ++q) {
+            const double zp = -fma(a[q], z, b[q] * zn) * rb[q];
+            zn = z;
+            z = zp;
+            nrm = fma(z, z, nrm);
+            if (q % 4 == 3) {  // an element grows by 2e14 at most (beta > 1e-14 |alpha|)
+                const double sc = nrm > 1e100 ? 1e-50 : 1.0;
+                z *= sc;
+                zn *= sc;
+                last *= sc;
+                nrm *= sc * sc;
+            }
         }
-        nrm = 1.0 / sqrt(nrm);
-        for (int i = 0; i < m; ++i) z[i] *= nrm;
     }
-    return z[m - 1];
+    return nrm < 1e300 ? last / sqrt(nrm) : 0.0;  // not finite: no residual
 }
 
 __device__ __forceinline__ double start_value(uint64_t seed, uint64_t q) {
@@ -117,203 +160,324 @@ __device__ __forceinline__ double start_value(uint64_t seed, uint64_t q) {
 
 }  // namespace
 
-// NT threads, rows tid + k * NT for k < R (n <= NT * R = MAXN).
-template <int NT, int R>
-__global__ void __launch_bounds__(NT) k_doci_batch_lanczos(const DociBatchJob* __restrict__ jobs) {
-    constexpr int MAXN = NT * R;
-    constexpr int NW = NT / 64;
-    __shared__ double x[MAXN];                       // v_j
-    __shared__ double hop[kBatchMaxL * kBatchMaxL];  // V(j,j,k,k)
-    __shared__ double pd[kBatchMaxL * kBatchMaxL];   // 2 (kk|ll) - (kl|lk), k != l
-    __shared__ double d1[kBatchMaxL];                // 2 h_ii + (ii|ii)
-    __shared__ double al[kMaxSteps], be[kMaxSteps];
-    __shared__ double wk[2 * kMaxSteps];
-    __shared__ double red[2][NW];
-    __shared__ double ctl[4];                        // beta, stop flag, theta0, res0
-    const DociBatchJob J = jobs[blockIdx.x];
+namespace {
+
+// Block sum over NT threads in a fixed order.
+template <int NT>
+__device__ __forceinline__ double block_sum(double v, double* red) {
+    v = wave_sum64(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) s += red[i];
+    __syncthreads();
+    return s;
+}
+
+// The parts of a request's scratch.
+struct Work {
+    double *dg, *u, *v, *al, *be, *hop;
+    __device__ explicit Work(const DociBatchJob& J) {
+        const size_t n = (size_t)J.n;
+        dg = J.scratch;
+        u = dg + n;
+        v = u + 2 * n;
+        al = v + 3 * n;
+        be = al + kMaxSteps + 2;
+        hop = be + kMaxSteps + 2;
+    }
+};
+
+// Convergence test of T_m by the whole workgroup (two waves work); sets the
+// request's result and done flag when it stops.
+__device__ void lanczos_test(const DociBatchJob& J, int m, int maxs, TestMatrix& T, int count, int* left, int* flag) {
+    const Work W(J);
+    __shared__ double ctl[6];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int L = J.L, np = J.np, nv = J.nv;
-    const int n = J.n;
-    for (int t = tid; t < L * L; t += NT) {
+    const double alpha = W.al[m - 1], beta = W.be[m - 1];
+    const bool broke = !(beta > 1e-14 * fabs(alpha));
+    if (!((m >= 4 && m % J.check == 0) || m == maxs || broke)) return;
+    double glo = 1e300, ghi = -1e300;  // Gershgorin bounds, in every wave
+    for (int i = lane; i < m; i += 64) {
+        const double rad = (i > 0 ? fabs(W.be[i - 1]) : 0.0) + (i < m - 1 ? fabs(W.be[i]) : 0.0);
+        glo = fmin(glo, W.al[i] - rad);
+        ghi = fmax(ghi, W.al[i] + rad);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        glo = fmin(glo, __shfl_xor(glo, off, 64));
+        ghi = fmax(ghi, __shfl_xor(ghi, off, 64));
+    }
+    const double pad = 1e-12 * fmax(1.0, fmax(fabs(glo), fabs(ghi)));
+    const double mid = 0.5 * (glo + ghi), half = 0.5 * (ghi - glo) + pad, rh = 1.0 / half;
+    for (int i = tid; i < (m + kBlk - 1) / kBlk * kBlk; i += blockDim.x) {
+        const double bl = i > 0 && i < m ? W.be[i - 1] * rh : 0.0;
+        T.a[i] = i < m ? (W.al[i] - mid) * rh : 4.0;
+        T.b2[i] = bl * bl;
+        const int q = m - 1 - i;  // row of element i counted from the end
+        const double bp = q > 0 ? W.be[q - 1] * rh : 0.0;
+        T.ra[i] = q >= 0 ? (W.al[q] - mid) * rh : 0.0;
+        T.rn[i] = i > 0 && q >= 0 ? W.be[q] * rh : 0.0;
+        T.rb[i] = bp != 0.0 ? 1.0 / bp : 0.0;
+    }
+    __syncthreads();
+    double* last_th = W.al + kMaxSteps;  // theta_0 and theta_1 of the last test
+    if (wv < 2 && wv < m) {  // theta_0 and theta_1 at the same time
+        const double xk = kth_eigenvalue(T, m, wv, (last_th[wv] - mid) * rh, 1e-13);
+        if (lane == 0) {
+            ctl[wv] = xk;
+            last_th[wv] = mid + half * xk;
+        }
+    }
+    __syncthreads();
+    const double x0 = ctl[0], th0 = mid + half * x0;
+    double x1 = m > 1 ? ctl[1] : x0;
+    bool have1 = m > 1;
+    int k1 = 1;
+    while (have1 && half * (x1 - x0) <= 1e-10 * fmax(1.0, fabs(th0))) {  // copies of theta_0 skipped
+        __syncthreads();
+        if (++k1 >= m || k1 >= 6) {
+            have1 = false;
+            break;
+        }
+        if (wv == 0) {
+            const double xk = kth_eigenvalue(T, m, k1, 2.0, 1e-13);
+            if (lane == 0) ctl[1] = xk;
+        }
+        __syncthreads();
+        x1 = ctl[1];
+    }
+    if (lane == 0 && wv < 2) ctl[2 + wv] = beta * last_component(T, m, wv == 0 ? x0 : x1);
+    __syncthreads();
+    const double r0 = ctl[2], r1 = ctl[3], th1 = mid + half * x1;
+    bool stop = r0 <= J.tol * fabs(th0) || broke;
+    if (!stop && J.tol_energy > 0.0 && have1) {
+        const double mu = th1 - r1;
+        stop = mu > th0 && r0 * r0 <= J.tol_energy * (mu - th0);
+    }
+    if ((stop || m == maxs) && wv == 0) {
+        const double xf = kth_eigenvalue(T, m, 0, x0, 1e-16);
+        if (lane == 0) {
+            J.out[0] = mid + half * xf;
+            J.out[1] = r0;
+            J.out[2] = (double)m;
+            J.out[3] = stop ? 0.0 : 1.0;
+            *J.done = 1;
+            if (atomicAdd(left, 1) + 1 == count) {
+                *flag = 1;  // host memory
+                __threadfence_system();
+            }
+        }
+    }
+}
+
+}  // namespace
+
+__global__ void __launch_bounds__(256) k_doci_hops(const str_t* __restrict__ s, uint64_t n, int L, int np,
+                                                   uint32_t* __restrict__ col) {
+    const uint64_t r = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= n) return;
+    const str_t full = L >= 64 ? ~(str_t)0 : ((str_t)1 << L) - 1;
+    str_t o = s[r];
+    const str_t vir = ~o & full;
+    uint64_t t = 0;
+    for (int a = 0; a < np; ++a) {
+        const int j = 63 - __builtin_clzll(o);
+        o ^= (str_t)1 << j;
+        for (str_t v = vir; v;) {
+            const int k = 63 - __builtin_clzll(v);
+            v ^= (str_t)1 << k;
+            uint32_t* e = col + t * n + r;
+            *e = (uint32_t)(j * L + k) << 20 | *e << 3;
+            ++t;
+        }
+    }
+}
+
+void launch_doci_hops(const str_t* s, uint64_t n, int L, int np, uint32_t* col, hipStream_t st) {
+    if (!n) return;
+    CF_REQUIRE(L <= kBatchMaxL && n <= (uint64_t)doci_batch_capacity(), "packed hops: L <= 32, n <= 13312");
+    k_doci_hops<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(s, n, L, np, col);
+    CF_HIP(hipGetLastError());
+}
+
+// Diagonal and hop elements of every request; the request is not done.
+__global__ void __launch_bounds__(256) k_doci_batch_init(const DociBatchJob* __restrict__ jobs, int* left) {
+    __shared__ double pd[kBatchMaxL * kBatchMaxL];  // 2 (kk|ll) - (kl|lk), k != l
+    __shared__ double d1[kBatchMaxL];               // 2 h_ii + (ii|ii)
+    const DociBatchJob J = jobs[blockIdx.y];
+    const Work W(J);
+    const int L = J.L;
+    if ((int)(blockIdx.x * 256) >= J.n) return;
+    for (int t = threadIdx.x; t < L * L; t += 256) {
         const int j = t / L, k = t - j * L;
         const int lo = j < k ? j : k, hi = j < k ? k : j;
-        hop[t] = J.V[(((size_t)lo * L + lo) * L + hi) * L + hi];
+        if (blockIdx.x == 0) W.hop[t] = J.V[(((size_t)lo * L + lo) * L + hi) * L + hi];
         pd[t] = j == k ? 0.0
                        : 2.0 * J.V[(((size_t)j * L + k) * L + j) * L + k] - J.V[(((size_t)j * L + k) * L + k) * L + j];
     }
-    for (int t = tid; t < L; t += NT) d1[t] = 2.0 * J.h[t * L + t] + J.V[(((size_t)t * L + t) * L + t) * L + t];
-    __syncthreads();
-    // this thread's rows r = tid, tid + NT, ...: diagonal, previous Krylov
-    // vector and w in the request's scratch (each row touched by one thread only)
-    double* dg = J.scratch;
-    double* vp = J.scratch + n;
-    double* w = J.scratch + 2 * (size_t)n;
-    double part = 0.0;
-    for (int r = tid; r < n; r += NT) {
-        const str_t s = J.s[r];
-        double e = 0.0;
-        for (str_t u = s; u; u &= u - 1) {
-            const int i = __builtin_ctzll(u);
-            e += d1[i];
-            for (str_t v = s; v; v &= v - 1) e += pd[i * L + __builtin_ctzll(v)];
-        }
-        dg[r] = e;
-        vp[r] = 0.0;
-        const double v0 = start_value(J.seed, (uint64_t)r);
-        w[r] = v0;
-        part += v0 * v0;
-    }
-    auto block_sum2 = [&](double a, double b, double* outa, double* outb) {
-        a = wave_sum64(a);
-        b = wave_sum64(b);
-        if (lane == 0) {
-            red[0][wv] = a;
-            red[1][wv] = b;
-        }
-        __syncthreads();
-        double sa = 0.0, sb = 0.0;
-        for (int i = 0; i < NW; ++i) {
-            sa += red[0][i];
-            sb += red[1][i];
-        }
-        *outa = sa;
-        *outb = sb;
-        __syncthreads();
-    };
-    double nrm2, dummy;
-    block_sum2(part, 0.0, &nrm2, &dummy);
-    {
-        const double sc = 1.0 / sqrt(nrm2);
-        for (int r = tid; r < n; r += NT) x[r] = w[r] * sc;
+    for (int t = threadIdx.x; t < L; t += 256)
+        d1[t] = 2.0 * J.h[t * L + t] + J.V[(((size_t)t * L + t) * L + t) * L + t];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *J.done = 0;
+        W.al[kMaxSteps] = W.al[kMaxSteps + 1] = 1e300;  // no test yet
+        if (blockIdx.y == 0) *left = 0;
     }
     __syncthreads();
-    const str_t full = ((str_t)1 << L) - 1;
-    double beta_prev = 0.0, theta0 = 0.0, res0 = 0.0;
-    int steps = 0, status = 1;
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= J.n) return;
+    const str_t s = J.s[r];
+    double e = 0.0;
+    for (str_t u = s; u; u &= u - 1) {
+        const int i = __builtin_ctzll(u);
+        e += d1[i];
+        for (str_t v = s; v; v &= v - 1) e += pd[i * L + __builtin_ctzll(v)];
+    }
+    W.dg[r] = e;
+}
+
+// Step j of every request: workgroups [0, nchunk) form v_j and H v_j on their
+// rows, workgroup nchunk tests T_{j-1}.  NT threads, rows tid + k NT of the
+// sums for k < R (n <= NT R).  Dynamic LDS: v_j and the hop elements.
+template <int NT, int R>
+__global__ void __launch_bounds__(NT) k_doci_batch_step(const DociBatchJob* __restrict__ jobs, int j, int nchunk,
+                                                        int count, int* left, int* flag) {
+    extern __shared__ __align__(16) unsigned char smem_batch[];
+    __shared__ double red[NT / 64];
+    const DociBatchJob& J = jobs[blockIdx.y];
+    if (*J.done) return;
     const int maxs = J.max_steps < kMaxSteps ? J.max_steps : kMaxSteps;
-    for (int j = 0; j < maxs; ++j) {
-        // w = H v_j
-        double pa = 0.0;
-        for (int r = tid; r < n; r += NT) {
-            const str_t s = J.s[r], vir = ~s & full;
-            const double xr = x[r];
-            double acc = dg[r] * xr;
-            const uint32_t* cp = J.col + r;
-            uint32_t t = 0;
-            str_t o = s;
-            for (int a = 0; a < np; ++a) {
-                const int jj = 63 - __builtin_clzll(o);
-                o ^= (str_t)1 << jj;
-                str_t v = vir;
-                for (int b = 0; b < nv; ++b) {
-                    const int kk = 63 - __builtin_clzll(v);
-                    v ^= (str_t)1 << kk;
-                    acc += hop[jj * L + kk] * x[cp[(size_t)t * n]];
-                    ++t;
-                }
-            }
-            w[r] = acc;
-            pa += xr * acc;
-        }
-        double alpha;
-        block_sum2(pa, 0.0, &alpha, &dummy);
-        double pb = 0.0;
-        for (int r = tid; r < n; r += NT) {
-            const double wr = w[r] - alpha * x[r] - beta_prev * vp[r];
-            w[r] = wr;
-            pb += wr * wr;
-        }
-        double b2;
-        block_sum2(pb, 0.0, &b2, &dummy);
-        const double beta = sqrt(b2);
-        if (tid == 0) {
-            al[j] = alpha;
-            be[j] = beta;
-        }
-        steps = j + 1;
-        // convergence test on T_{j+1} (wave 0)
-        const bool test = (j + 1 >= 4 && (j + 1) % J.check == 0) || j + 1 == maxs || !(beta > 1e-14 * fabs(alpha));
-        if (test) {
-            __syncthreads();
-            if (wv == 0) {
-                const int m = j + 1;
-                // Gershgorin bracket
-                double glo = 1e300, ghi = -1e300;
-                for (int i = lane; i < m; i += 64) {
-                    const double rad = (i > 0 ? fabs(be[i - 1]) : 0.0) + (i < m - 1 ? fabs(be[i]) : 0.0);
-                    glo = fmin(glo, al[i] - rad);
-                    ghi = fmax(ghi, al[i] + rad);
-                }
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) {
-                    glo = fmin(glo, __shfl_xor(glo, off, 64));
-                    ghi = fmax(ghi, __shfl_xor(ghi, off, 64));
-                }
-                const double pad = 1e-12 * fmax(1.0, fmax(fabs(glo), fabs(ghi)));
-                glo -= pad;
-                ghi += pad;
-                const double th0 = kth_eigenvalue(al, be, m, 0, glo, ghi);
-                double th1 = 0.0;
-                int k1 = 1;
-                bool have1 = false;
-                for (; k1 < m && k1 < 6; ++k1) {  // next distinct value (copies of theta0 skipped)
-                    th1 = kth_eigenvalue(al, be, m, k1, glo, ghi);
-                    if (th1 - th0 > 1e-10 * fmax(1.0, fabs(th0))) {
-                        have1 = true;
-                        break;
-                    }
-                }
-                if (lane == 0) {
-                    const double z0 = last_component(al, be, m, th0, wk);
-                    const double r0 = fabs(beta * z0);
-                    double r1 = 0.0;
-                    if (have1) r1 = fabs(beta * last_component(al, be, m, th1, wk));
-                    bool stop = r0 <= J.tol * fabs(th0) || !(beta > 1e-14 * fabs(alpha));
-                    if (!stop && J.tol_energy > 0.0 && have1) {
-                        const double mu = th1 - r1;
-                        stop = mu > th0 && r0 * r0 <= J.tol_energy * (mu - th0);
-                    }
-                    ctl[1] = stop ? 1.0 : 0.0;
-                    ctl[2] = th0;
-                    ctl[3] = r0;
-                }
-            }
-            __syncthreads();
-            theta0 = ctl[2];
-            res0 = ctl[3];
-            if (ctl[1] != 0.0) {
-                status = 0;
-                break;
-            }
-        }
-        if (j + 1 == maxs) break;
-        // v_{j+1} = w / beta; v_j kept in registers
-        __syncthreads();  // every gather of v_j is done
-        const double inv = 1.0 / beta;
-        for (int r = tid; r < n; r += NT) {
-            vp[r] = x[r];
-            x[r] = w[r] * inv;
-        }
-        beta_prev = beta;
-        __syncthreads();
+    if ((int)blockIdx.x == nchunk) {
+        if (j >= 2 && j - 1 <= maxs) lanczos_test(J, j - 1, maxs, *(TestMatrix*)smem_batch, count, left, flag);
+        return;
     }
-    if (tid == 0) {
-        J.out[0] = theta0;
-        J.out[1] = res0;
-        J.out[2] = (double)steps;
-        J.out[3] = (double)status;
+    const int n = J.n, L = J.L, tid = threadIdx.x;
+    const int rows = ((n + nchunk - 1) / nchunk + 63) / 64 * 64, r0 = (int)blockIdx.x * rows;
+    if (j > maxs || r0 >= n) return;
+    const Work W(J);
+    double* x = (double*)smem_batch;
+    double* hop = x + n;
+    for (int t = tid; t < L * L; t += NT) hop[t] = W.hop[t];
+    double w[R];
+    double part = 0.0;
+    if (j == 0) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int r = tid + k * NT;
+            w[k] = r < n ? start_value(J.seed, (uint64_t)r) : 0.0;
+            part += w[k] * w[k];
+        }
+    } else {
+        const double* u = W.u + (size_t)((j - 1) & 1) * n;
+        const double* v = W.v + (size_t)((j + 2) % 3) * n;
+        const double* vp = W.v + (size_t)((j + 1) % 3) * n;
+        double vj[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int r = tid + k * NT;
+            w[k] = r < n ? u[r] : 0.0;
+            vj[k] = r < n ? v[r] : 0.0;
+        }
+        double vq[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int r = tid + k * NT;
+            vq[k] = j > 1 && r < n ? vp[r] : 0.0;
+        }
+        const double beta_prev = j > 1 ? W.be[j - 2] : 0.0;
+        double pa = 0.0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) pa += vj[k] * w[k];
+        const double alpha = block_sum<NT>(pa, red);
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            w[k] = w[k] - alpha * vj[k] - beta_prev * vq[k];
+            part += w[k] * w[k];
+        }
+        if (blockIdx.x == 0 && tid == 0) W.al[j - 1] = alpha;
+    }
+    const double beta = sqrt(block_sum<NT>(part, red));
+    if (j > 0 && blockIdx.x == 0 && tid == 0) W.be[j - 1] = beta;
+    if (j == maxs) return;  // T_maxs is complete
+    const double inv = 1.0 / beta;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int r = tid + k * NT;
+        if (r < n) x[r] = w[k] * inv;
+    }
+    __syncthreads();
+    double* vout = W.v + (size_t)(j % 3) * n;
+    double* uout = W.u + (size_t)(j & 1) * n;
+    const int nh = J.np * J.nv;
+    const unsigned char* xb = (const unsigned char*)x;
+    const unsigned char* hb = (const unsigned char*)hop;
+    const int re = r0 + rows < n ? r0 + rows : n;
+    for (int r = r0 + tid; r < re; r += NT) {
+        const double xr = x[r];
+        vout[r] = xr;
+        double acc = W.dg[r] * xr;
+        const uint32_t* cp = J.hops + r;
+        int t = 0;
+        for (; t + 8 <= nh; t += 8) {
+            uint32_t e[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) e[q] = cp[(size_t)(t + q) * n];
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                acc = fma(*(const double*)(hb + (e[q] >> 17)), *(const double*)(xb + (e[q] & 0x1ffffu)), acc);
+        }
+        for (; t < nh; ++t) {
+            const uint32_t e = cp[(size_t)t * n];
+            acc = fma(*(const double*)(hb + (e >> 17)), *(const double*)(xb + (e & 0x1ffffu)), acc);
+        }
+        uout[r] = acc;
     }
 }
 
 int doci_batch_capacity() { return 1024 * 13; }
 
-void launch_doci_batch_lanczos(const DociBatchJob* d_jobs, int count, int max_n, hipStream_t s) {
-    if (count <= 0) return;
-    if (max_n <= 1024) k_doci_batch_lanczos<256, 4><<<(unsigned)count, 256, 0, s>>>(d_jobs);
-    else if (max_n <= 4096) k_doci_batch_lanczos<512, 8><<<(unsigned)count, 512, 0, s>>>(d_jobs);
-    else if (max_n <= 1024 * 13) k_doci_batch_lanczos<1024, 13><<<(unsigned)count, 1024, 0, s>>>(d_jobs);
-    else throw Error(ERR_UNSUPPORTED, "batched DOCI solve: more than 13,312 determinants");
+namespace {
+template <int NT, int R>
+void run_class(const DociBatchJob* d_jobs, int count, int max_n, int max_L, int max_steps, int* left,
+               volatile int* flag, hipEvent_t ev[2], hipStream_t s) {
+    const size_t lds = std::max(((size_t)max_n + (size_t)max_L * max_L) * sizeof(double), sizeof(TestMatrix));
+    CF_HIP(hipFuncSetAttribute((const void*)k_doci_batch_step<NT, R>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+    // enough workgroups to fill the GPU, none with less than a row a thread
+    const int nchunk = std::max(1, std::min((max_n + NT - 1) / NT, (1024 + count - 1) / count));
+    int* dflag = nullptr;
+    CF_HIP(hipHostGetDevicePointer((void**)&dflag, const_cast<int*>(flag), 0));
+    *flag = 0;
+    k_doci_batch_init<<<dim3((unsigned)((max_n + 255) / 256), (unsigned)count), 256, 0, s>>>(d_jobs, left);
     CF_HIP(hipGetLastError());
+    constexpr int kAhead = 8;
+    const int last = max_steps + 2;  // launches 0 .. max_steps + 1
+    for (int j = 0, g = 0; j < last; ++g) {
+        for (int e = std::min(last, j + kAhead); j < e; ++j) {
+            k_doci_batch_step<NT, R><<<dim3((unsigned)nchunk + 1, (unsigned)count), NT, lds, s>>>(
+                d_jobs, j, nchunk, count, left, dflag);
+            CF_HIP(hipGetLastError());
+        }
+        CF_HIP(hipEventRecord(ev[g & 1], s));
+        if (g > 0) {
+            CF_HIP(hipEventSynchronize(ev[(g - 1) & 1]));
+            if (*flag) break;
+        }
+    }
+    // what is still queued writes `flag` and the requests' scratch: the
+    // caller reads the results and reuses both only after it has run
+    CF_HIP(hipStreamSynchronize(s));
+}
+}  // namespace
+
+void run_doci_batch(const DociBatchJob* d_jobs, int count, int max_n, int max_L, int max_steps, int* left,
+                    volatile int* flag, hipEvent_t ev[2], hipStream_t s) {
+    if (count <= 0) return;
+    if (max_n <= 1024) run_class<256, 4>(d_jobs, count, max_n, max_L, max_steps, left, flag, ev, s);
+    else if (max_n <= 4096) run_class<512, 8>(d_jobs, count, max_n, max_L, max_steps, left, flag, ev, s);
+    else if (max_n <= 1024 * 13) run_class<1024, 13>(d_jobs, count, max_n, max_L, max_steps, left, flag, ev, s);
+    else throw Error(ERR_UNSUPPORTED, "batched DOCI solve: more than 13,312 determinants");
 }
 
 }  // namespace cf

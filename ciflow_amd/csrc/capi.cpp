@@ -2301,7 +2301,7 @@ int cf_rdm(cf_space* sp, const double* cvec, double* one, double* two) {
     API_END
 }
 
-// Batched small DOCI solves (one workgroup per request, see batch.hip).
+// Batched small DOCI solves (lock-step Lanczos, see batch.hip).
 int cf_solve_doci_batch(cf_ctx* ctx, int count, const cf_request* reqs, cf_result* results) {
     API_BEGIN
     CF_REQUIRE(ctx && (count == 0 || (reqs && results)), "NULL argument");
@@ -2381,12 +2381,14 @@ int cf_solve_doci_batch(cf_ctx* ctx, int count, const cf_request* reqs, cf_resul
         a.nv = L - np;
         a.s = T.s.p;
         launch_doci_ell_fill(a, ctx->binom.p, T.col.p, st);
+        launch_doci_hops(T.s.p, n, L, np, T.col.p, st);
     }
-    // jobs by size class: one launch each
+    // jobs by size class: one lock-step batch each
     uint64_t scratch_n = 0;
     for (int i = 0; i < count; ++i)
-        if (ok[i]) scratch_n += 3 * results[i].n;
+        if (ok[i]) scratch_n += doci_batch_scratch(results[i].n, reqs[i].L);
     DBuf<double> scratch(std::max<uint64_t>(scratch_n, 1)), dout(4 * (size_t)count);
+    DBuf<int> done((size_t)count + 1);
     std::vector<DociBatchJob> jobs;
     std::vector<int> order;
     uint64_t off = 0;
@@ -2405,13 +2407,14 @@ int cf_solve_doci_batch(cf_ctx* ctx, int count, const cf_request* reqs, cf_resul
             J.V = vptr[i];
             const cf_ctx::DociTables& T = ctx->doci_tabs[std::make_pair(r.L, r.nup)];
             J.s = T.s.p;
-            J.col = T.col.p;
+            J.hops = T.col.p;
             J.tol = r.tol > 0 ? r.tol : dflt.tol;
             J.tol_energy = r.tol_energy > 0 ? r.tol_energy : 0.0;
             J.seed = dflt.seed;
             J.out = dout.p + 4 * (size_t)i;
             J.scratch = scratch.p + off;
-            off += 3 * (uint64_t)n;
+            off += doci_batch_scratch((uint64_t)n, r.L);
+            J.done = done.p + i;
             J.L = r.L;
             J.np = r.nup;
             J.nv = r.L - r.nup;
@@ -2427,9 +2430,24 @@ int cf_solve_doci_batch(cf_ctx* ctx, int count, const cf_request* reqs, cf_resul
     DBuf<DociBatchJob> djobs(std::max<size_t>(jobs.size(), 1));
     if (!jobs.empty())
         CF_HIP(hipMemcpyAsync(djobs.p, jobs.data(), jobs.size() * sizeof(DociBatchJob), hipMemcpyHostToDevice, st));
+    hipEvent_t ev[2] = {ctx->event(), ctx->event()};
+    ctx->pool.reserve(ctx->pool.size() + 2);
+    struct Events {  // back to the context's events also when a launch throws
+        cf_ctx* c;
+        hipEvent_t* e;
+        ~Events() { c->pool.insert(c->pool.end(), e, e + 2); }
+    } keep{ctx, ev};
     for (int c = 0; c < 3; ++c) {
         const size_t a = ranges[c].first, b = ranges[c].second;
-        if (b > a) launch_doci_batch_lanczos(djobs.p + a, (int)(b - a), bounds[c], st);
+        if (b == a) continue;
+        int max_n = 0, max_L = 0, max_steps = 0;
+        for (size_t q = a; q < b; ++q) {
+            max_n = std::max(max_n, jobs[q].n);
+            max_L = std::max(max_L, jobs[q].L);
+            max_steps = std::max(max_steps, jobs[q].max_steps);
+        }
+        run_doci_batch(djobs.p + a, (int)(b - a), max_n, max_L, max_steps, done.p + count,
+                       (volatile int*)(ctx->pinned + 255), ev, st);
     }
     std::vector<double> hout(4 * (size_t)count, 0.0);
     CF_HIP(hipMemcpyAsync(hout.data(), dout.p, hout.size() * sizeof(double), hipMemcpyDeviceToHost, st));

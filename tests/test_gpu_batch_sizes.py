@@ -1,0 +1,47 @@
+"""GPU tests of cf_solve_doci_batch at the edges of its workgroup shapes and
+splits: spaces of 2 to 13,312 rows around the three shapes' bounds, more
+requests than fill the GPU, tight tolerances (many steps) and a step limit
+that ends a solve, each against dense eigenvalues or the stored-matrix solve."""
+import numpy as np
+import pytest
+
+import ciflow_amd as CA
+
+pytestmark = pytest.mark.gpu
+
+
+def request(L, npair, seed):
+    h, V = CA.gen_integrals(L, seed)
+    return {"h": h, "V": V, "npair": npair, "U": CA.expm_skew(CA.gen_rotation(L, seed, 0.05))}
+
+
+def stored_energy(q):
+    h, V = CA.rotate_integrals(q["h"], q["V"], q["U"])
+    ci = CA.DOCI(CA.Hamiltonian(h, V, q["npair"], q["npair"]))
+    if ci.n <= 1001:
+        row, col, val = ci.get_mat().export_full()
+        A = np.zeros((ci.n, ci.n))
+        for i in range(ci.n):
+            A[i, col[row[i]:row[i + 1]]] = val[row[i]:row[i + 1]]
+        return np.linalg.eigvalsh(A)[0]
+    ci.solve()
+    return ci.get_ci_energy()
+
+
+@pytest.mark.parametrize("L,npair", [(2, 1), (4, 2), (8, 4), (12, 6), (14, 4), (13, 8), (14, 7), (15, 6), (16, 8),
+                                     (32, 1), (28, 2)])
+def test_batch_sizes(L, npair):
+    q = request(L, npair, 40 + L + npair)
+    res = CA.solve_doci_batch([dict(q), dict(q, tol=1e-9), dict(q, tol_energy=1e-9)])
+    E = stored_energy(q)
+    for r, tol in zip(res, (1e-10, 1e-9, 1e-8)):
+        assert r["status"] == 0 and r["solve_status"] == 0
+        assert abs(r["energy"] - E) <= tol, (r["n"], r["n_matvec"], r["energy"], E)
+
+
+def test_more_requests_than_workgroups_fill_the_gpu():
+    qs = [request(10, 5, 500 + k) for k in range(4)]
+    alone = [CA.solve_doci_batch([q])[0] for q in qs]
+    res = CA.solve_doci_batch([qs[k % 4] for k in range(1100)])   # one workgroup per request
+    for k, r in enumerate(res):
+        assert r["energy"] == alone[k % 4]["energy"] and r["n_matvec"] == alone[k % 4]["n_matvec"]
