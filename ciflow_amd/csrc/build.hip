@@ -27,6 +27,8 @@
 // offsets of these segments; a lane finds its segment by binary search.
 #include "kernels.h"
 
+#include <algorithm>
+
 #include <hipcub/hipcub.hpp>
 #include "string_ops.h"
 
@@ -36,25 +38,36 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-__global__ void k_fci_segoff(uint64_t da, int Ea, const Exc* __restrict__ full_a, int Eb, int Sb,
-                             uint32_t* __restrict__ segoff) {
-    uint64_t ia = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (ia >= da) return;
+// One wavefront per alpha string: lengths of 64 entries at a time, scanned.
+__global__ void __launch_bounds__(64) k_fci_segoff(uint64_t da, int Ea, const Exc* __restrict__ full_a, int Eb, int Sb,
+                                                   uint32_t* __restrict__ segoff) {
+    const uint64_t ia = blockIdx.x;
+    const int lane = threadIdx.x;
     const Exc* lst = full_a + ia * (uint64_t)Ea;
     uint32_t* so = segoff + ia * (uint64_t)(Ea + 1);
-    uint32_t acc = 0;
-    for (int e = 0; e < Ea; ++e) {
-        so[e] = acc;
-        int t = lst[e].type;
-        acc += t == 0 ? (uint32_t)Eb : (t == 1 ? (uint32_t)Sb : 1u);
+    uint32_t base = 0;
+    for (int e0 = 0; e0 < Ea; e0 += 64) {
+        const int e = e0 + lane;
+        uint32_t v = 0;
+        if (e < Ea) {
+            const int t = lst[e].type;
+            v = t == 0 ? (uint32_t)Eb : t == 1 ? (uint32_t)Sb : 1u;
+        }
+        uint32_t inc = v;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += o;
+        }
+        if (e < Ea) so[e] = base + inc - v;
+        base += __shfl(inc, 63, 64);
     }
-    so[Ea] = acc;
+    if (lane == 0) so[Ea] = base;
 }
 
 void launch_fci_segoff(uint64_t da, int Ea, const Exc* full_a, int Eb, int Sb, uint32_t* segoff,
                        hipStream_t stream) {
     if (!da) return;
-    k_fci_segoff<<<(unsigned)((da + 255) / 256), 256, 0, stream>>>(da, Ea, full_a, Eb, Sb, segoff);
+    k_fci_segoff<<<(unsigned)da, 64, 0, stream>>>(da, Ea, full_a, Eb, Sb, segoff);
     CF_HIP(hipGetLastError());
 }
 
@@ -192,42 +205,255 @@ __global__ void __launch_bounds__(256) k_fci_rows(FciRowsArgs a) {
     if (!FILL && lane == 0) a.rowcnt[r - a.row0] = cnt;
 }
 
-// Position-major copy of the complete FCI rows of one alpha string:
-// ell[(ia*R + t)*db + ib] = element t of row (ia, ib), 0 where the element is
-// not stored (|v| <= zero).  One thread per beta string, so the writes of a
-// wavefront are contiguous.
-__global__ void __launch_bounds__(256) k_fci_ell(FciRowsArgs a, uint32_t chunks, double* __restrict__ ell,
-                                                 float* __restrict__ ell32) {
-    const uint64_t ia = blockIdx.x / chunks;
-    const uint64_t ib = (uint64_t)(blockIdx.x - ia * chunks) * 256 + threadIdx.x;
-    if (ia >= a.da || ib >= a.db) return;
-    const str_t Sa = a.sa[ia], Sb = a.sb[ib];
+// ---------------------------------------------------------------------------
+// FCI rows in two steps (d_beta <= 65535).  k_fci_ell evaluates every element
+// once, position-major -- ell[((ia - ia0) R + t) db + ib] = element t of row (ia,
+// ib), 0 where it is not stored (|v| <= zero) -- and counts each row's stored
+// elements on the way; k_fci_crs then writes the CRS rows from it through LDS
+// tiles.  Evaluating per row, as k_fci_rows does, costs a binary search and a
+// chain of list and integral loads per element, twice (count and fill), and
+// the position-major copy a third time from lists read 16 bytes per lane at a
+// stride: 1.53 + 1.85 + 2.05 ms for the 1.8e8 elements of FCI L=11 5a4b against
+// 0.56 ms (1.43 GB of values, 2.6 TB/s) + 1.29 ms (3.6 GB read and written, 2.8
+// TB/s) now.  k_fci_rows stays for d_beta > 65535, whose targets need 32 bits.
+//
+// In k_fci_ell a workgroup owns one alpha string and a chunk of beta strings
+// (one a thread), and a part of the positions.  The beta lists come from
+// position-major tables (coalesced u16 codes, f L + t and the phase in bit 15);
+// an alpha single's V slice and W row sit in LDS (double-buffered, one barrier a
+// single), so an element is one u16 load, one LDS read, a sign and a coalesced
+// store: bound by the stores.
+// ---------------------------------------------------------------------------
+constexpr uint16_t kBetaSelf = 0xffff, kBetaSingle = 0x4000, kBetaSign = 0x8000, kBetaPair = 0x0fff;
+
+__global__ void k_beta_tables(uint64_t db, int L, int Sb, int Eb, const Exc* __restrict__ subb,
+                              const Exc* __restrict__ fullb, uint16_t* __restrict__ jsub, uint16_t* __restrict__ jfull,
+                              uint16_t* __restrict__ csub, uint16_t* __restrict__ cfull, double* __restrict__ xfull) {
+    // consecutive threads take consecutive strings: coalesced writes
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= db * (uint64_t)(Sb + Eb)) return;
+    const uint64_t u = t / db, ib = t - u * db;
+    const bool sub = u < (uint64_t)Sb;
+    const uint64_t v = sub ? u : u - Sb;
+    const Exc e = sub ? subb[ib * Sb + v] : fullb[ib * Eb + v];
+    const uint16_t code = e.type == 0 ? kBetaSelf
+                                      : (uint16_t)((e.f * L + e.t) | (e.type == 1 ? kBetaSingle : 0) |
+                                                   (e.sign < 0 ? kBetaSign : 0));
+    (sub ? jsub : jfull)[v * db + ib] = (uint16_t)e.J;
+    (sub ? csub : cfull)[v * db + ib] = code;
+    if (!sub) xfull[v * db + ib] = e.x;
+}
+
+void launch_beta_tables(uint64_t db, int L, int Sb, int Eb, const Exc* subb, const Exc* fullb, uint16_t* jsub,
+                        uint16_t* jfull, uint16_t* csub, uint16_t* cfull, double* xfull, hipStream_t s) {
+    if (db > 65535 || L > 64) throw Error(ERR_UNSUPPORTED, "beta tables need d_beta <= 65535 and L <= 64");
+    const uint64_t tot = db * (uint64_t)(Eb + Sb);
+    if (!tot) return;
+    k_beta_tables<<<(unsigned)((tot + 255) / 256), 256, 0, s>>>(db, L, Sb, Eb, subb, fullb, jsub, jfull, csub, cfull,
+                                                              xfull);
+    CF_HIP(hipGetLastError());
+}
+
+__device__ __forceinline__ double with_sign(double v, bool neg) {
+    return __hiloint2double(__double2hiint(v) ^ (neg ? (int)0x80000000 : 0), __double2loint(v));
+}
+
+__global__ void __launch_bounds__(512) k_fci_ell(FciEllArgs A, uint32_t chunks, uint32_t rows) {
+    extern __shared__ double smem_ell[];
+    const FciRowsArgs& a = A.r;
+    const int L = a.H.L, L2 = L * L, tid = threadIdx.x;
+    const uint64_t db = a.db;
+    const uint64_t il = blockIdx.x / chunks, ia = A.ia0 + il;
+    const uint32_t chunk = blockIdx.x - (uint32_t)(il * chunks);
+    const uint64_t ib = (uint64_t)chunk * rows + tid;
+    const bool act = (uint32_t)tid < rows && ib < db;
+    const uint64_t ibs = act ? ib : 0;
+    const str_t Sa = a.sa[ia], Sb = a.sb[ibs];
     const uint32_t* so = a.segoff + ia * (uint64_t)(a.Ea + 1);
-    const uint64_t R = so[a.Ea];
+    const uint32_t R = so[a.Ea];
     const Exc* la = a.fa + ia * (uint64_t)a.Ea;
-    const Exc* lb = a.fb + ib * (uint64_t)a.Eb;
-    const Exc* sbl = a.subb + ib * (uint64_t)a.Sb;
-    for (int k = 0; k < a.Ea; ++k) {
+    double* ell = A.ell ? A.ell + il * R * db + ibs : nullptr;
+    float* ell32 = A.ell32 ? A.ell32 + il * R * db + ibs : nullptr;
+    // this part's alpha entries: those that begin in [lo, hi)
+    auto first_at = [&](uint32_t t) {
+        int lo = 0, hi = a.Ea;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (so[mid] < t) lo = mid + 1;
+            else hi = mid;
+        }
+        return lo;
+    };
+    const int k0 = first_at((uint32_t)((uint64_t)R * blockIdx.y / gridDim.y));
+    const int k1 = first_at((uint32_t)((uint64_t)R * (blockIdx.y + 1) / gridDim.y));
+    uint32_t cnt = 0;
+    auto put = [&](uint32_t t, double v) {
+        const bool keep = fabs(v) > a.zero;
+        if (!keep) v = 0.0;
+        if (act) {
+            cnt += keep ? 1u : 0u;
+            if (ell) __builtin_nontemporal_store(v, ell + (uint64_t)t * db);
+            if (ell32) __builtin_nontemporal_store((float)v, ell32 + (uint64_t)t * db);
+        }
+    };
+    int buf = 0;
+    for (int k = k0; k < k1; ++k) {
         const Exc ea = la[k];
-        const uint32_t len = so[k + 1] - so[k];
-        for (uint32_t u = 0; u < len; ++u) {
-            uint32_t col;
-            double val;
-            fci_entry(a, ia, ib, Sa, Sb, ea, lb, sbl, u, col, val);
-            if (!(fabs(val) > a.zero)) val = 0.0;
-            const uint64_t pos = (ia * R + so[k] + u) * a.db + ib;
-            if (ell) ell[pos] = val;
-            if (ell32) ell32[pos] = (float)val;
+        const uint32_t t0 = so[k];
+        if (ea.type == 2) {
+            put(t0, ea.x);
+        } else if (ea.type == 1) {
+            double* Vs = smem_ell + buf * (L2 + L);
+            double* Ws = Vs + L2;
+            buf ^= 1;
+            const int f = ea.f, t = ea.t;
+            const double* w = a.H.W + ((size_t)(f < t ? f : t) * L + (f < t ? t : f)) * L;
+            for (int i = tid; i < L2 + L; i += blockDim.x) {
+                if (i >= L2) {
+                    Ws[i - L2] = w[i - L2];
+                } else {  // orientation of the reference's upper entry
+                    const int q = i / L, r = i - q * L;
+                    Vs[i] = ea.J > ia ? a.H.V[(((size_t)f * L + q) * L + t) * L + r]
+                                      : a.H.V[(((size_t)t * L + r) * L + f) * L + q];
+                }
+            }
+            __syncthreads();
+            const bool neg = ea.sign < 0;
+            double self = ea.x;
+            for (str_t b = Sb; b; b &= b - 1) self += Ws[__builtin_ctzll(b)];
+            if (neg) self *= -1;
+            const uint16_t* cs = A.csub + ibs;
+#pragma unroll 8
+            for (int u = 0; u < a.Sb; ++u) {
+                const uint32_t c = cs[(uint64_t)u * db];
+                const double v = with_sign(Vs[c == kBetaSelf ? 0 : c & kBetaPair], neg != ((c & kBetaSign) != 0));
+                put(t0 + u, c == kBetaSelf ? self : v);
+            }
+        } else {
+            const uint16_t* cf_ = A.cfull + ibs;
+            const double* xf = A.xfull + ibs;
+#pragma unroll 4
+            for (int u = 0; u < a.Eb; ++u) {
+                const uint32_t c = cf_[(uint64_t)u * db];
+                double v = xf[(uint64_t)u * db];
+                if (c == kBetaSelf) {
+                    v = a.diag[ia * db + ibs];
+                } else if (c & kBetaSingle) {
+                    const int f = (int)(c & kBetaPair) / L, t = (int)(c & kBetaPair) - f * L;
+                    const double* w = a.H.W + ((size_t)(f < t ? f : t) * L + (f < t ? t : f)) * L;
+                    for (str_t s = Sa; s; s &= s - 1) v += w[__builtin_ctzll(s)];
+                    if (c & kBetaSign) v *= -1;
+                }
+                put(t0 + u, v);
+            }
+        }
+    }
+    if (A.rowcnt && act) atomicAdd(&A.rowcnt[ia * db + ib], cnt);
+}
+
+void launch_fci_ell(const FciEllArgs& A, hipStream_t stream) {
+    const FciRowsArgs& a = A.r;
+    if (!A.nia || !a.db) return;
+    if (A.rowcnt) CF_HIP(hipMemsetAsync(A.rowcnt + A.ia0 * a.db, 0, A.nia * a.db * sizeof(uint32_t), stream));
+    const uint64_t chunks = (a.db + 511) / 512;
+    const uint32_t rows = (uint32_t)((a.db + chunks - 1) / chunks);
+    const unsigned nt = (rows + 63) / 64 * 64;
+    if (A.nia * chunks > 0x7fffffffull) throw Error(ERR_UNSUPPORTED, "FCI element grid too large");
+    // parts of the positions where the strings alone make fewer than 16,384 waves
+    const uint64_t waves = A.nia * chunks * (nt / 64);
+    const unsigned parts = (unsigned)std::min<uint64_t>(8, std::max<uint64_t>(1, 16384 / waves));
+    const size_t lds = 2 * (size_t)(a.H.L * a.H.L + a.H.L) * sizeof(double);
+    if (lds > 64 * 1024)
+        CF_HIP(hipFuncSetAttribute((const void*)k_fci_ell, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    k_fci_ell<<<dim3((unsigned)(A.nia * chunks), parts), nt, lds, stream>>>(A, (uint32_t)chunks, rows);
+    CF_HIP(hipGetLastError());
+}
+
+// CRS rows of alpha strings [ia0, ia0 + nia) from their position-major values:
+// a workgroup takes 64 beta strings of one alpha string, 64 positions at a time
+// through an LDS tile (values and beta targets read along the strings, rows
+// written along the positions), zeros left out.
+__global__ void __launch_bounds__(256) k_fci_crs(FciRowsArgs a, uint64_t ia0, const double* __restrict__ ell,
+                                                 const uint16_t* __restrict__ jsub, const uint16_t* __restrict__ jfull,
+                                                 uint32_t tiles) {
+    __shared__ double tv[64][65];
+    __shared__ uint16_t tj[64][66];
+    __shared__ uint32_t jbase[64];
+    __shared__ int32_t jrow[64];  // row of jsub (>= 0), ~row of jfull (< -1), -1: the string itself
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t db = a.db;
+    const uint64_t il = blockIdx.x / tiles, ia = ia0 + il;
+    const uint64_t ib0 = (uint64_t)(blockIdx.x - (uint32_t)(il * tiles)) * 64;
+    const uint32_t* so = a.segoff + ia * (uint64_t)(a.Ea + 1);
+    const uint32_t R = so[a.Ea];
+    const Exc* la = a.fa + ia * (uint64_t)a.Ea;
+    const bool actb = ib0 + lane < db;
+    int64_t base[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const uint64_t ib = ib0 + w * 16 + q;
+        base[q] = ib < db ? a.rowptr[ia * db + ib] : 0;
+    }
+    for (uint32_t t0 = 0; t0 < R; t0 += 64) {
+        __syncthreads();  // the last tile has been written out
+        if (threadIdx.x < 64 && t0 + lane < R) {
+            const uint32_t t = t0 + lane;
+            int lo = 0, hi = a.Ea;  // largest e with so[e] <= t
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (so[mid] <= t) lo = mid;
+                else hi = mid;
+            }
+            const Exc ea = la[lo];
+            const int u = (int)(t - so[lo]);
+            jbase[lane] = (uint32_t)((ea.type == 0 ? ia : (uint64_t)ea.J) * db);
+            jrow[lane] = ea.type == 0 ? -2 - u : ea.type == 1 ? u : -1;
+        }
+        __syncthreads();
+        double v[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const uint32_t t = t0 + w * 16 + q;
+            v[q] = actb && t < R ? __builtin_nontemporal_load(ell + (il * R + t) * db + ib0 + lane) : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int tt = w * 16 + q, jr = jrow[tt];
+            uint16_t j = (uint16_t)(ib0 + lane);
+            if (actb && t0 + tt < R) {
+                if (jr >= 0) j = jsub[(uint64_t)jr * db + ib0 + lane];
+                else if (jr < -1) j = jfull[(uint64_t)(-2 - jr) * db + ib0 + lane];
+            }
+            tj[tt][lane] = j;
+            tv[tt][lane] = v[q];
+        }
+        __syncthreads();
+        const bool actt = t0 + lane < R;
+        const uint32_t jb = actt ? jbase[lane] : 0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int r = w * 16 + q;
+            if (ib0 + r >= db) break;
+            const double v = actt ? tv[lane][r] : 0.0;
+            const bool keep = v != 0.0;
+            const uint64_t mask = __ballot(keep);
+            if (keep) {
+                const int64_t pos = base[q] + lanes_below(mask);
+                a.col[pos] = jb + tj[lane][r];
+                a.val[pos] = v;
+                if (a.val32) a.val32[pos] = (float)v;
+            }
+            base[q] += __popcll(mask);
         }
     }
 }
 
-void launch_fci_ell(const FciRowsArgs& a, double* ell, float* ell32, hipStream_t stream) {
-    const uint64_t chunks = (a.db + 255) / 256;
-    const uint64_t grid = a.da * chunks;
-    if (!grid) return;
-    if (grid > 0xffffffffull) throw Error(ERR_UNSUPPORTED, "ELL build grid too large");
-    k_fci_ell<<<(unsigned)grid, 256, 0, stream>>>(a, (uint32_t)chunks, ell, ell32);
+void launch_fci_crs(const FciRowsArgs& a, uint64_t ia0, uint64_t nia, const double* ell, const uint16_t* jsub,
+                    const uint16_t* jfull, hipStream_t stream) {
+    const uint64_t tiles = (a.db + 63) / 64;
+    if (!nia || !tiles) return;
+    if (nia * tiles > 0x7fffffffull) throw Error(ERR_UNSUPPORTED, "FCI row grid too large");
+    k_fci_crs<<<(unsigned)(nia * tiles), 256, 0, stream>>>(a, ia0, ell, jsub, jfull, (uint32_t)tiles);
     CF_HIP(hipGetLastError());
 }
 

@@ -135,7 +135,7 @@ struct cf_crs {
     DBuf<uint16_t> jsub, jfull;
     DBuf<uint2> ent;
     EllArgs eargs;
-    bool ell_ready = false;
+    bool ell_ready = false;  // tables and values
     // DOCI position-major hop columns + pair tables (kernel 5)
     DBuf<uint32_t> dcol;
     DBuf<double> dvk;
@@ -435,26 +435,67 @@ void make_doci_blocks(cf_crs* m, int w) {
     m->blk_ready = true;
 }
 
-// Position-major complete FCI rows + beta index tables (kernel 4).
-void make_ell(cf_crs* m) {
+// Position-major beta tables of an FCI space for its current Hamiltonian.
+struct BetaTables {
+    DBuf<uint16_t> jsub, jfull, csub, cfull;
+    DBuf<double> xfull;
+    explicit BetaTables(const cf_space* sp) {
+        const StrTab* tb = sp->tb;
+        const uint64_t ns = (uint64_t)tb->S * sp->db, nf = (uint64_t)tb->E * sp->db;
+        jsub.alloc(ns);
+        csub.alloc(ns);
+        jfull.alloc(nf);
+        cfull.alloc(nf);
+        xfull.alloc(nf);
+        launch_beta_tables(sp->db, sp->ham->L, tb->S, tb->E, tb->sub.p, tb->full.p, jsub.p, jfull.p, csub.p, cfull.p,
+                           xfull.p, sp->ham->ctx->stream);
+    }
+};
+
+// Positions of one row.
+uint64_t fci_row_length(const cf_space* sp) {
+    const int Ea = sp->ta->E, Sb = sp->tb->S, Eb = sp->tb->E;
+    const int nsa = sp->ta->S - 1, nda = Ea - 1 - nsa;
+    return (uint64_t)Eb + (uint64_t)nsa * Sb + nda;
+}
+
+// Evaluates the rows of alpha strings [ia0, ia0 + nia) position-major.
+void eval_fci_rows(cf_crs* m, const FciRowsArgs& fa, const BetaTables& T, uint64_t ia0, uint64_t nia, double* ell,
+                   float* ell32, uint32_t* rowcnt) {
+    FciEllArgs e{};
+    e.r = fa;
+    e.csub = T.csub.p;
+    e.cfull = T.cfull.p;
+    e.xfull = T.xfull.p;
+    e.ia0 = ia0;
+    e.nia = nia;
+    e.ell = ell;
+    e.ell32 = ell32;
+    e.rowcnt = rowcnt;
+    launch_fci_ell(e, m->sp->ham->ctx->stream);
+}
+
+// Position-major complete FCI rows + beta index tables (kernel 4); counts each
+// row's stored elements into rowcnt (may be null).
+void make_ell(cf_crs* m, uint32_t* rowcnt = nullptr) {
     cf_space* sp = m->sp;
     cf_ctx* c = sp->ham->ctx;
     CF_REQUIRE(sp->kind == CF_FCI && m->has_fargs, "the ELL SpMV needs an FCI matrix");
     CF_REQUIRE(sp->db <= kEllMaxDb, "the ELL SpMV needs d_beta <= 8192");
     const int Ea = sp->ta->E, Sb = sp->tb->S, Eb = sp->tb->E;
     const int nsa = sp->ta->S - 1, nda = Ea - 1 - nsa;
-    const uint64_t R = (uint64_t)Eb + (uint64_t)nsa * Sb + nda;
-    m->jsub.alloc((uint64_t)Sb * sp->db);
-    m->jfull.alloc((uint64_t)Eb * sp->db);
-    launch_ell_index(sp->db, Sb, Eb, sp->tb->sub.p, sp->tb->full.p, m->jsub.p, m->jfull.p, c->stream);
+    const uint64_t R = fci_row_length(sp);
+    BetaTables T(sp);
     m->ent.alloc(sp->da * (uint64_t)Ea);
     launch_ell_entries(sp->da, Ea, nda, nsa, sp->ta->full.p, sp->segoff.p, m->ent.p, c->stream);
     m->ell.alloc(m->n * R);
     if (m->want32) m->ell32.alloc(m->n * R);
     {
         KTimer t(c, "crs_fill");
-        launch_fci_ell(m->fargs, m->ell.p, m->ell32.p, c->stream);
+        eval_fci_rows(m, m->fargs, T, 0, sp->da, m->ell.p, m->ell32.p, rowcnt);
     }
+    m->jsub = std::move(T.jsub);
+    m->jfull = std::move(T.jfull);
     EllArgs& e = m->eargs;
     e.da = sp->da;
     e.db = sp->db;
@@ -471,6 +512,12 @@ void make_ell(cf_crs* m) {
     e.R = R;
     m->ell_ready = true;
 }
+
+// FCI matrices with enough alpha strings to fill the GPU get the
+// position-major copy (kernel 4): measured 2.38 ms against 5.15 ms (FP64) and
+// 1.53 ms against 3.45 ms (FP32) at L = 12, 0.52 / 0.90 ms at L = 11; at
+// L = 10 (252 alpha strings) the row gather stays faster
+bool wants_ell(const cf_space* sp) { return sp->kind == CF_FCI && sp->da >= 400 && sp->db <= kEllMaxDb; }
 
 // Staged FCI SpMV plan (alpha-block structure of the rows).
 void make_fci_plan(cf_crs* m, int W) {
@@ -512,6 +559,11 @@ void build_crs_arrays(cf_crs* m) {
     // determinant lists with L <= 32 find each row's columns by excitation
     // lookup in the sorted (up, down) keys instead of n^2 pair tests
     const bool lookup = sp->kind == CF_DETS && H->L <= 32;
+    // FCI rows with 16-bit beta targets are written from their position-major values
+    const bool from_values = sp->kind == CF_FCI && sp->db <= 65535;
+    std::unique_ptr<BetaTables> tabs;
+    DBuf<double> values;
+    uint64_t piece = sp->da;  // alpha strings per pass of the values
     DBuf<uint64_t> skey;
     DBuf<uint32_t> sidx;
     DetLookupArgs largs{};
@@ -560,8 +612,23 @@ void build_crs_arrays(cf_crs* m) {
         m->fargs = fa;
         m->fargs.rowcnt = nullptr;
         m->has_fargs = true;
-        KTimer t(c, "crs_count");
-        launch_fci_rows(fa, false, c->stream);
+        if (from_values && wants_ell(sp) && !m->ell_ready) {
+            make_ell(m, cnt.p);
+        } else if (from_values) {
+            KTimer t(c, "crs_count");
+            tabs.reset(new BetaTables(sp));
+            if (!m->ell_ready) {  // the values pass through a buffer of at most 2 GiB
+                const uint64_t per = fci_row_length(sp) * sp->db;
+                piece = std::min<uint64_t>(sp->da, std::max<uint64_t>(1, (2ull << 30) / (per * sizeof(double))));
+                values.alloc(piece * per);
+            }
+            for (uint64_t i = 0; i < sp->da; i += piece)
+                eval_fci_rows(m, fa, *tabs, i, std::min(piece, sp->da - i), m->ell_ready ? m->ell.p : values.p,
+                              m->ell_ready ? m->ell32.p : nullptr, cnt.p);
+        } else {
+            KTimer t(c, "crs_count");
+            launch_fci_rows(fa, false, c->stream);
+        }
     } else {
         dargs.d = sp->n;
         dargs.L = H->L;
@@ -607,7 +674,17 @@ void build_crs_arrays(cf_crs* m) {
         fa.val = m->val.p;
         fa.val32 = m->val32.p;
         KTimer t(c, "crs_fill");
-        launch_fci_rows(fa, true, c->stream);
+        if (m->ell_ready && from_values) {
+            launch_fci_crs(fa, 0, sp->da, m->ell.p, m->jsub.p, m->jfull.p, c->stream);
+        } else if (from_values) {
+            for (uint64_t i = 0; i < sp->da; i += piece) {
+                const uint64_t k = std::min(piece, sp->da - i);
+                if (piece < sp->da) eval_fci_rows(m, fa, *tabs, i, k, values.p, nullptr, nullptr);
+                launch_fci_crs(fa, i, k, values.p, tabs->jsub.p, tabs->jfull.p, c->stream);
+            }
+        } else {
+            launch_fci_rows(fa, true, c->stream);
+        }
     } else {
         dargs.rowptr = m->rowptr.p;
         dargs.col = m->col.p;
@@ -636,7 +713,8 @@ void sync_ham(cf_crs* m) {
     if (m->has_fargs) m->fargs.H = H;
     if (m->ell_ready) {
         KTimer t(c, "crs_fill");
-        launch_fci_ell(m->fargs, m->ell.p, m->ell32.p, c->stream);
+        const BetaTables T(sp);
+        eval_fci_rows(m, m->fargs, T, 0, sp->da, m->ell.p, m->ell32.p, nullptr);
     }
     m->plan.reset();  // the staged kernel reads the CRS arrays; rebuilt on request
     m->sell_ready = false;  // the sliced copy too, after the CRS arrays
@@ -1184,12 +1262,8 @@ int cf_crs_build(cf_space* sp, int value_prec, double zero, cf_crs** out) {
     if (avg >= 512) m->auto64 = SpmvChoice{3, 16, 2, {}, {}};
     if (avg >= 128) m->auto32 = SpmvChoice{3, 8, 2, {}, {}};
     else if (avg >= 24) m->auto32 = SpmvChoice{3, 16, 1, {}, {}};
-    // FCI matrices with enough alpha strings to fill the GPU also get the
-    // position-major copy (kernel 4): measured 2.38 ms against 5.15 ms (FP64) and
-    // 1.53 ms against 3.45 ms (FP32) at L = 12, 0.52 / 0.90 ms at L = 11; at
-    // L = 10 (252 alpha strings) the row gather stays faster
-    if (sp->kind == CF_FCI && sp->da >= 400 && sp->db <= kEllMaxDb) {
-        make_ell(m.get());
+    if (wants_ell(sp)) {
+        if (!m->ell_ready) make_ell(m.get());  // made with the CRS arrays where these come from it
         m->auto64 = SpmvChoice{4, 0, 0, ell_default_shape(sp->db, 8), {}};
         m->auto32 = SpmvChoice{4, 0, 0, ell_default_shape(sp->db, 4), {}};
     }

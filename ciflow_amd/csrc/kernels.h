@@ -66,9 +66,27 @@ struct FciRowsArgs {
     float* val32;
 };
 void launch_fci_rows(const FciRowsArgs& a, bool fill, hipStream_t stream);
-// Position-major (per alpha string) copy of the complete rows, zeros where
-// |v| <= zero; either output may be null.
-void launch_fci_ell(const FciRowsArgs& a, double* ell, float* ell32, hipStream_t stream);
+// Position-major beta tables of an FCI space: targets j, codes and full-list
+// values x of entry u of string ib at [u * db + ib] (db <= 65535).
+void launch_beta_tables(uint64_t db, int L, int Sb, int Eb, const Exc* subb, const Exc* fullb, uint16_t* jsub,
+                        uint16_t* jfull, uint16_t* csub, uint16_t* cfull, double* xfull, hipStream_t s);
+struct FciEllArgs {
+    FciRowsArgs r;
+    const uint16_t* csub;   // launch_beta_tables
+    const uint16_t* cfull;
+    const double* xfull;
+    uint64_t ia0, nia;      // alpha strings of this launch
+    double* ell;            // [nia][R][db] (either may be null)
+    float* ell32;
+    uint32_t* rowcnt;       // stored elements of each row of the whole space (null: not counted)
+};
+// Position-major (per alpha string) values of the complete rows, zeros where
+// |v| <= zero.
+void launch_fci_ell(const FciEllArgs& a, hipStream_t stream);
+// CRS rows (col, val, val32 by rowptr) of alpha strings [ia0, ia0 + nia) from
+// their position-major values.
+void launch_fci_crs(const FciRowsArgs& a, uint64_t ia0, uint64_t nia, const double* ell, const uint16_t* jsub,
+                    const uint16_t* jfull, hipStream_t stream);
 
 struct DociRowsArgs {
     uint64_t d;

@@ -34,9 +34,6 @@ void launch_ell_entries(uint64_t da, int Ea, int nda, int nsa, const Exc* fa, co
 // Default shape for a beta dimension and value size (4 or 8 bytes).
 EllShape ell_default_shape(uint64_t db, int value_bytes);
 
-// jsub[u*db + ib] = sub(ib)[u].J, jfull[u*db + ib] = full(ib)[u].J (db <= 65535).
-void launch_ell_index(uint64_t db, int Sb, int Eb, const Exc* subb, const Exc* fullb, uint16_t* jsub,
-                      uint16_t* jfull, hipStream_t s);
 // Largest beta dimension the LDS-staged kernel supports.
 constexpr uint64_t kEllMaxDb = 8192;
 void launch_spmv_ell_f64(const EllArgs& a, EllShape sh, const double* ell, const double* x, double* y,

@@ -21,30 +21,6 @@
 
 namespace cf {
 
-__global__ void k_ell_index(uint64_t db, int Sb, int Eb, const Exc* __restrict__ subb,
-                            const Exc* __restrict__ fullb, uint16_t* __restrict__ jsub,
-                            uint16_t* __restrict__ jfull) {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t ns = db * (uint64_t)Sb, nf = db * (uint64_t)Eb;
-    if (t < ns) {
-        const uint64_t ib = t / Sb, u = t - ib * Sb;
-        jsub[u * db + ib] = (uint16_t)subb[t].J;
-    }
-    if (t < nf) {
-        const uint64_t ib = t / Eb, u = t - ib * Eb;
-        jfull[u * db + ib] = (uint16_t)fullb[t].J;
-    }
-}
-
-void launch_ell_index(uint64_t db, int Sb, int Eb, const Exc* subb, const Exc* fullb, uint16_t* jsub,
-                      uint16_t* jfull, hipStream_t s) {
-    if (db > 65535) throw Error(ERR_UNSUPPORTED, "ELL index tables need d_beta <= 65535");
-    const uint64_t tot = db * (uint64_t)(Eb > Sb ? Eb : Sb);
-    if (!tot) return;
-    k_ell_index<<<(unsigned)((tot + 255) / 256), 256, 0, s>>>(db, Sb, Eb, subb, fullb, jsub, jfull);
-    CF_HIP(hipGetLastError());
-}
-
 template <typename VT>
 __device__ __forceinline__ double ldv(const VT* p) {
     return (double)__builtin_nontemporal_load(p);
@@ -121,26 +97,27 @@ __global__ void __launch_bounds__(NT) k_spmv_ell(EllArgs a, uint32_t chunks, con
 // thread owns beta strings (ib, ib+1) and reads their values, indices and x
 // entries with paired loads (VEC = 4: four strings, 16/32-byte loads).
 // ---------------------------------------------------------------------------
-__global__ void k_ell_entries(uint64_t da, int Ea, int nda, int nsa, const Exc* __restrict__ fa,
-                              const uint32_t* __restrict__ segoff, uint2* __restrict__ ent) {
-    const uint64_t ia = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (ia >= da) return;
+// One wavefront per alpha string, 64 entries at a time.
+__global__ void __launch_bounds__(64) k_ell_entries(uint64_t da, int Ea, int nda, int nsa, const Exc* __restrict__ fa,
+                                                    const uint32_t* __restrict__ segoff, uint2* __restrict__ ent) {
+    const uint64_t ia = blockIdx.x;
+    const int lane = threadIdx.x;
     const Exc* la = fa + ia * (uint64_t)Ea;
     const uint32_t* so = segoff + ia * (uint64_t)(Ea + 1);
     uint2* e = ent + ia * (uint64_t)Ea;
     int d = 0, sg = 0;
-    for (int k = 0; k < Ea; ++k) {
-        const uint2 w = make_uint2(so[k], la[k].J);
-        const int ty = la[k].type;
-        if (ty == 2) {
-            if (d < nda) e[d] = w;
-            ++d;
-        } else if (ty == 1) {
-            if (sg < nsa) e[nda + sg] = w;
-            ++sg;
-        } else {
-            e[nda + nsa] = w;
+    for (int k0 = 0; k0 < Ea; k0 += 64) {
+        const int k = k0 + lane;
+        const int ty = k < Ea ? la[k].type : -1;
+        const uint64_t md = __ballot(ty == 2), ms = __ballot(ty == 1), below = ((uint64_t)1 << lane) - 1;
+        if (ty >= 0) {
+            const int at = ty == 2   ? d + __popcll(md & below)
+                           : ty == 1 ? nda + sg + __popcll(ms & below)
+                                     : nda + nsa;
+            if (at < Ea) e[at] = make_uint2(so[k], la[k].J);
         }
+        d += __popcll(md);
+        sg += __popcll(ms);
     }
 }
 
@@ -148,7 +125,7 @@ void launch_ell_entries(uint64_t da, int Ea, int nda, int nsa, const Exc* fa, co
                         hipStream_t s) {
     if (!da) return;
     if (nda + nsa + 1 != Ea) throw Error(ERR_STATE, "ELL entries: alpha list counts do not add up");
-    k_ell_entries<<<(unsigned)((da + 255) / 256), 256, 0, s>>>(da, Ea, nda, nsa, fa, segoff, ent);
+    k_ell_entries<<<(unsigned)da, 64, 0, s>>>(da, Ea, nda, nsa, fa, segoff, ent);
     CF_HIP(hipGetLastError());
 }
 

@@ -191,11 +191,14 @@ __global__ void __launch_bounds__(64) k_exc_lists(int L, int nel, const str_t* _
     }
     __syncthreads();
     // self + singles sub-list, keeps the sorted order
-    if (lane == 0) {
-        Exc* so = sub + idx * (uint64_t)S;
-        int w = 0;
-        for (int e = 0; e < E && w < S; ++e)
-            if (out[e].type != 2) so[w++] = out[e];
+    Exc* so = sub + idx * (uint64_t)S;
+    int w = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + lane;
+        const bool in = e < E && (code[e] & 3u) != 2u;
+        const uint64_t mask = __ballot(in);
+        if (in) so[w + __popcll(mask & (((uint64_t)1 << lane) - 1))] = out[e];
+        w += __popcll(mask);
     }
 }
 
