@@ -34,10 +34,6 @@
 
 namespace cf {
 
-__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
 // One wavefront per alpha string: lengths of 64 entries at a time, scanned.
 __global__ void __launch_bounds__(64) k_fci_segoff(uint64_t da, int Ea, const Exc* __restrict__ full_a, int Eb, int Sb,
                                                    uint32_t* __restrict__ segoff) {
@@ -69,17 +65,6 @@ void launch_fci_segoff(uint64_t da, int Ea, const Exc* full_a, int Eb, int Sb, u
     if (!da) return;
     k_fci_segoff<<<(unsigned)da, 64, 0, stream>>>(da, Ea, full_a, Eb, Sb, segoff);
     CF_HIP(hipGetLastError());
-}
-
-// jmix of CIMethod::diagonal (CIMethod.cpp:343-351): sum over alpha k (outer),
-// beta l (inner), accumulated from zero.
-__device__ __forceinline__ double jmix(str_t a, str_t b, const HamDev& H) {
-    double s = 0.0;
-    for (str_t t = a; t; t &= t - 1) {
-        int k = __builtin_ctzll(t);
-        for (str_t u = b; u; u &= u - 1) s += H.Jm[k * H.L + __builtin_ctzll(u)];
-    }
-    return s;
 }
 
 __global__ void k_fci_diag(uint64_t da, uint64_t db, const str_t* __restrict__ sa, const str_t* __restrict__ sb,
@@ -853,20 +838,20 @@ void sort_det_keys(uint64_t n, const str_t* up, const str_t* down, uint64_t* ske
 }
 
 // Each row's (col, val) pairs sorted by column (rows given by rowptr).
-void sort_rows_by_column(uint64_t n, uint64_t nnz, const int64_t* rowptr, uint32_t* col, double* val,
+void sort_rows_by_column(uint64_t n, uint64_t nnz, const int64_t* rowptr, DBuf<uint32_t>& col, DBuf<double>& val,
                          hipStream_t stream) {
     if (!nnz) return;
     if (nnz > 0x7fffffffull || n > 0x7fffffffull) throw Error(ERR_UNSUPPORTED, "row sort: too many entries");
     DBuf<uint32_t> col2(nnz);
     DBuf<double> val2(nnz);
     size_t tb = 0;
-    CF_HIP(hipcub::DeviceSegmentedRadixSort::SortPairs(nullptr, tb, col, col2.p, val, val2.p, (int)nnz, (int)n,
+    CF_HIP(hipcub::DeviceSegmentedRadixSort::SortPairs(nullptr, tb, col.p, col2.p, val.p, val2.p, (int)nnz, (int)n,
                                                        rowptr, rowptr + 1, 0, 32, stream));
     DBuf<unsigned char> tmp(tb);
-    CF_HIP(hipcub::DeviceSegmentedRadixSort::SortPairs(tmp.p, tb, col, col2.p, val, val2.p, (int)nnz, (int)n,
+    CF_HIP(hipcub::DeviceSegmentedRadixSort::SortPairs(tmp.p, tb, col.p, col2.p, val.p, val2.p, (int)nnz, (int)n,
                                                        rowptr, rowptr + 1, 0, 32, stream));
-    CF_HIP(hipMemcpyAsync(col, col2.p, nnz * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream));
-    CF_HIP(hipMemcpyAsync(val, val2.p, nnz * sizeof(double), hipMemcpyDeviceToDevice, stream));
+    col = std::move(col2);
+    val = std::move(val2);
 }
 
 void launch_det_rows(const DetRowsArgs& a, bool fill, hipStream_t stream) {

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "capi_types.h"
+#include "dets.h"
 #include "kernels.h"
 #include "host.h"
 #include "lanczos.h"
@@ -335,8 +336,8 @@ bool make_sell(cf_crs* m, bool optional = false) {
     }
     if (!m->spart.p && m->n < (1ull << 21)) m->spart.alloc(kSellMaxSplit * m->n);
     KTimer t(c, "crs_fill");
-    launch_sell_fill(m->n, m->rowptr.p, m->col.p, m->val.p, m->want32 ? m->val32.p : nullptr, m->sqoff.p, m->scol.p,
-                     m->sval.p, m->want32 ? m->sval32.p : nullptr, c->stream);
+    launch_sell_fill(m->n, m->rowptr.p, m->col.p, m->val.p, m->sqoff.p, m->scol.p, m->sval.p,
+                     m->want32 ? m->sval32.p : nullptr, c->stream);
     CF_HIP(hipStreamSynchronize(c->stream));
     m->sell_ready = true;
     return true;
@@ -567,6 +568,8 @@ void build_crs_arrays(cf_crs* m) {
     DBuf<uint64_t> skey;
     DBuf<uint32_t> sidx;
     DetLookupArgs largs{};
+    DetTables dtabs;
+    bool tables = false;
     if (sp->kind == CF_DETS) {
         targs.n = sp->n;
         targs.nup = H->nup;
@@ -585,7 +588,9 @@ void build_crs_arrays(cf_crs* m) {
             largs.sidx = sidx.p;
             largs.L = H->L;
             KTimer t(c, "crs_count");
-            launch_det_rows_lookup(largs, false, c->stream);
+            tables = make_det_tables(dtabs, sp->n, sp->dup.p, sp->ddown.p, skey.p, sidx.p, H->dev(), c->stream);
+            if (tables) launch_det_rows_tab(dtabs, targs, false, c->stream);
+            else launch_det_rows_lookup(largs, false, c->stream);
         } else {
             KTimer t(c, "crs_count");
             launch_det_rows(targs, false, c->stream);
@@ -657,13 +662,22 @@ void build_crs_arrays(cf_crs* m) {
         targs.val = m->val.p;
         targs.val32 = m->val32.p;
         KTimer t(c, "crs_fill");
-        if (lookup && m->nnz <= 0x7fffffffull) {
+        const bool in_order = sp->ascending + 1 >= sp->n;  // the tables' rows are sorted then
+        targs.rowcnt = nullptr;
+        if (tables && (in_order || m->nnz <= 0x7fffffffull)) {
+            if (!in_order) targs.val32 = nullptr;
+            launch_det_rows_tab(dtabs, targs, true, c->stream);
+            if (!in_order) {
+                sort_rows_by_column(m->n, m->nnz, m->rowptr.p, m->col, m->val, c->stream);
+                if (m->want32) launch_to_f32(m->nnz, m->val.p, m->val32.p, c->stream);
+            }
+        } else if (lookup && m->nnz <= 0x7fffffffull) {
             largs.r.rowcnt = nullptr;
             largs.r.rowptr = m->rowptr.p;
             largs.r.col = m->col.p;
             largs.r.val = m->val.p;
             launch_det_rows_lookup(largs, true, c->stream);
-            sort_rows_by_column(m->n, m->nnz, m->rowptr.p, m->col.p, m->val.p, c->stream);
+            sort_rows_by_column(m->n, m->nnz, m->rowptr.p, m->col, m->val, c->stream);
             if (m->want32) launch_to_f32(m->nnz, m->val.p, m->val32.p, c->stream);
         } else {
             launch_det_rows(targs, true, c->stream);

@@ -136,7 +136,7 @@ void launch_det_sigma_lookup(const DetLookupArgs& a, const double* x, double* y,
 // bits: significant key bits (32 + L)
 void sort_det_keys(uint64_t n, const str_t* up, const str_t* down, uint64_t* skey, uint32_t* sidx, int bits,
                    hipStream_t stream);
-void sort_rows_by_column(uint64_t n, uint64_t nnz, const int64_t* rowptr, uint32_t* col, double* val,
+void sort_rows_by_column(uint64_t n, uint64_t nnz, const int64_t* rowptr, DBuf<uint32_t>& col, DBuf<double>& val,
                          hipStream_t stream);
 
 // Exclusive scan of 32-bit counts into 64-bit offsets (n+1 entries).
@@ -172,8 +172,8 @@ void launch_spmv_sell_f32(uint64_t n, const int64_t* qoff, const uint32_t* col, 
 // Chunked copy of CRS rows: quads of each chunk's longest row, then the fill
 // (val32 / sval32 may be NULL).
 void launch_sell_quads(uint64_t n, const int64_t* rowptr, uint32_t* quads, hipStream_t stream);
-void launch_sell_fill(uint64_t n, const int64_t* rowptr, const uint32_t* col, const double* val, const float* val32,
-                      const int64_t* qoff, uint32_t* scol, double* sval, float* sval32, hipStream_t stream);
+void launch_sell_fill(uint64_t n, const int64_t* rowptr, const uint32_t* col, const double* val, const int64_t* qoff,
+                      uint32_t* scol, double* sval, float* sval32, hipStream_t stream);
 
 // Krylov vector kernels (vectors are columns of a column-major n x k block).
 void launch_multi_dot(uint64_t n, int k, const double* Vb, const double* w, double* partial, int nblocks,

@@ -374,37 +374,60 @@ __global__ void __launch_bounds__(256) k_sell_quads(uint64_t n, uint32_t nchunk,
     if (lane == 0) quads[c] = (len + 3) / 4;
 }
 
-// Copies the CRS rows into the sliced layout: one workgroup per chunk, wave
-// w writes quads w, w + 4, ... of the chunk's 64 rows.
+// Copies the CRS rows into the sliced layout: one workgroup per chunk of 64
+// rows, 64 entries of every row at a time through LDS, so the rows are read
+// along their entries and the quads written along the rows (lanes that each
+// walked a row of their own read 4 and 8 bytes per line: 1.72 against 0.70 ms for
+// 4.2e7 entries).
 __global__ void __launch_bounds__(256) k_sell_fill(uint64_t n, uint32_t nchunk, const int64_t* __restrict__ rowptr,
                                                    const uint32_t* __restrict__ col, const double* __restrict__ val,
-                                                   const float* __restrict__ val32, const int64_t* __restrict__ qoff,
+                                                   const int64_t* __restrict__ qoff,
                                                    uint32_t* __restrict__ scol, double* __restrict__ sval,
                                                    float* __restrict__ sval32) {
+    __shared__ double tv[64][65];
+    __shared__ uint32_t tc[64][65];
     const uint32_t c = blockIdx.x;
     if (c >= nchunk) return;
-    const int lane = threadIdx.x & 63;
-    const uint64_t r = (uint64_t)c * 64 + lane;
-    const int64_t s = r < n ? rowptr[r] : 0;
-    const int64_t len = r < n ? rowptr[r + 1] - s : 0;
-    const uint32_t pad = r < n ? (uint32_t)r : 0u;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t r0 = (uint64_t)c * 64;
     const int64_t q0 = qoff[c], nq = qoff[c + 1] - q0;
-    for (int64_t q = threadIdx.x >> 6; q < nq; q += 4) {
-        u32x4 cc;
-        f64x4 vv;
-        f32x4 ww;
+    // this wave's rows r0 + w + 4 k: start and length
+    int64_t s[16];
+    int len[16];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t k = 4 * q + j;
-            const bool in = k < len;
-            cc[j] = in ? col[s + k] : pad;
-            vv[j] = in ? val[s + k] : 0.0;
-            ww[j] = in && val32 ? val32[s + k] : 0.0f;
+    for (int k = 0; k < 16; ++k) {
+        const uint64_t r = r0 + w + 4 * k;
+        s[k] = r < n ? rowptr[r] : 0;
+        len[k] = r < n ? (int)(rowptr[r + 1] - s[k]) : 0;
+    }
+    for (int64_t e0 = 0; e0 < 4 * nq; e0 += 64) {
+        __syncthreads();  // the last tile has been written out
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int row = w + 4 * k;
+            const bool in = e0 + lane < len[k];
+            tc[row][lane] = in ? col[s[k] + e0 + lane] : r0 + row < n ? (uint32_t)(r0 + row) : 0u;
+            tv[row][lane] = in ? val[s[k] + e0 + lane] : 0.0;
         }
-        const uint64_t o = (uint64_t)(q0 + q) * 64 + lane;
-        ((u32x4*)scol)[o] = cc;
-        ((f64x4*)sval)[o] = vv;
-        if (sval32) ((f32x4*)sval32)[o] = ww;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int q = w + 4 * k;  // quad of the tile; lane = row
+            if (e0 / 4 + q >= nq) break;
+            u32x4 cc;
+            f64x4 vv;
+            f32x4 ww;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                cc[j] = tc[lane][4 * q + j];
+                vv[j] = tv[lane][4 * q + j];
+                ww[j] = (float)vv[j];  // val32 is the rounded value
+            }
+            const uint64_t o = (uint64_t)(q0 + e0 / 4 + q) * 64 + lane;
+            ((u32x4*)scol)[o] = cc;
+            ((f64x4*)sval)[o] = vv;
+            if (sval32) ((f32x4*)sval32)[o] = ww;
+        }
     }
 }
 
@@ -415,12 +438,11 @@ void launch_sell_quads(uint64_t n, const int64_t* rowptr, uint32_t* quads, hipSt
     CF_HIP(hipGetLastError());
 }
 
-void launch_sell_fill(uint64_t n, const int64_t* rowptr, const uint32_t* col, const double* val, const float* val32,
-                      const int64_t* qoff, uint32_t* scol, double* sval, float* sval32, hipStream_t stream) {
+void launch_sell_fill(uint64_t n, const int64_t* rowptr, const uint32_t* col, const double* val, const int64_t* qoff,
+                      uint32_t* scol, double* sval, float* sval32, hipStream_t stream) {
     const uint64_t nchunk = (n + 63) / 64;
     if (!nchunk) return;
-    k_sell_fill<<<(unsigned)nchunk, 256, 0, stream>>>(n, (uint32_t)nchunk, rowptr, col, val, val32, qoff, scol, sval,
-                                                      sval32);
+    k_sell_fill<<<(unsigned)nchunk, 256, 0, stream>>>(n, (uint32_t)nchunk, rowptr, col, val, qoff, scol, sval, sval32);
     CF_HIP(hipGetLastError());
 }
 

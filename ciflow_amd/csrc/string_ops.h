@@ -48,4 +48,19 @@ __device__ __forceinline__ int stacked(str_t common, int p, int q) {
     return __popcll(common & mask);
 }
 
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// jmix of CIMethod::diagonal (CIMethod.cpp:343-351): sum over alpha k (outer),
+// beta l (inner), accumulated from zero.
+__device__ __forceinline__ double jmix(str_t a, str_t b, const HamDev& H) {
+    double s = 0.0;
+    for (str_t t = a; t; t &= t - 1) {
+        int k = __builtin_ctzll(t);
+        for (str_t u = b; u; u &= u - 1) s += H.Jm[k * H.L + __builtin_ctzll(u)];
+    }
+    return s;
+}
+
 }  // namespace cf
