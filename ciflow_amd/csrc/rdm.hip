@@ -217,6 +217,7 @@ __global__ void k_sum_chunks(int nchunk, uint64_t len, const double* __restrict_
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= len) return;
     double s = 0.0;
+#pragma unroll 8
     for (int c = 0; c < nchunk; ++c) s += part[(uint64_t)c * len + i];
     out[i] = s;
 }
@@ -246,6 +247,29 @@ __global__ void k_doci_rdm(uint64_t d, int L, const str_t* __restrict__ s, const
         o[bin] = D;
         o[L2 + bin] = Pj;
         if (j == k) o[2 * L2 + j] = D;
+    }
+}
+
+__global__ void __launch_bounds__(256) k_zero(uint64_t n, double* __restrict__ out) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) out[i] = 0.0;
+}
+
+// Gamma[b][p][q][r][t] from the Gram blocks aa, ab, bb ([rp][qt]).
+static void unpack_gram(int L, const double* const blocks[3], const double* gamma, double* Gamma) {
+    const int P = L * L;
+    const size_t L4 = (size_t)P * P;
+    for (int b = 0; b < 3; ++b) {
+        const double* Gb = blocks[b];
+        const int s = b == 2 ? 1 : 0;
+        for (int p = 0; p < L; ++p)
+            for (int q = 0; q < L; ++q)
+                for (int r = 0; r < L; ++r)
+                    for (int t = 0; t < L; ++t) {
+                        double v = Gb[(size_t)(r * L + p) * P + (q * L + t)];
+                        if (b != 1 && q == r) v -= gamma[s * P + p * L + t];
+                        Gamma[b * L4 + (((size_t)p * L + q) * L + r) * L + t] = v;
+                    }
     }
 }
 
@@ -283,33 +307,356 @@ static void rdm_from_x(hipStream_t stream, int L, uint64_t n, const double* c, c
     std::vector<double> hG(3 * PP);
     CF_HIP(hipMemcpyAsync(hG.data(), G.p, 3 * PP * sizeof(double), hipMemcpyDeviceToHost, stream));
     CF_HIP(hipStreamSynchronize(stream));
-    const size_t L4 = PP;
-    for (int b = 0; b < 3; ++b) {
-        const double* Gb = hG.data() + b * PP;
-        const int s = b == 2 ? 1 : 0;
-        for (int p = 0; p < L; ++p)
-            for (int q = 0; q < L; ++q)
-                for (int r = 0; r < L; ++r)
-                    for (int t = 0; t < L; ++t) {
-                        double v = Gb[(size_t)(r * L + p) * P + (q * L + t)];
-                        if (b != 1 && q == r) v -= gamma[s * P + p * L + t];
-                        Gamma[b * L4 + (((size_t)p * L + q) * L + r) * L + t] = v;
-                    }
+    const double* blocks[3] = {hG.data(), hG.data() + PP, hG.data() + 2 * PP};
+    unpack_gram(L, blocks, gamma, Gamma);
+}
+
+// ---------------------------------------------------------------------------
+// FCI densities from one-spin matrices (L <= 16, string spaces of <= 16,384).
+//
+// For a fixed alpha string ka the transition densities X^a(ka, kb)_rp = s
+// c(J, kb) are rows of C with the string J = ka - r + p and the same for every
+// kb, so the same-spin part needs no Gram product over determinants: with
+//   M^a = C C^T (alpha strings),  M^b = C^T C (beta strings)
+//   gamma^a_rp         = sum_ka s M^a(ka, J_rp)
+//   sum_K X^a_rp X^a_qs = sum_ka s s' M^a(J_rp, J_qs),
+// 2 d^2 (d' ) flop and a gather instead of 2 n L^4.  The opposite-spin part
+//   sum_kb X^a_rp(ka, kb) X^b_qs(ka, kb)
+// is, per ka, a product of the na (L - na + 1) rows of C that X^a has (of L^2)
+// with X^b(ka, .), which is scattered into LDS from C's row ka: 24 instead of 64
+// MFMA tiles a step at L=11, nothing stored but each ka's block.  Blocks are
+// summed over ka in order.
+//
+// FCI L=11 5a5b (213,444 determinants): the L^2 columns of X built in memory
+// (0.24 + 0.06 ms), three Gram products over them (0.53 ms each) and two
+// weighted sums (0.42 ms each) took 3.2 ms a call; now 0.47 ms, of which
+// k_gram_ab 0.19 (2.6 GFLOP with the padding, 14 TFLOP/s: the scatter into LDS and
+// its barriers), the one-spin matrices 0.03 and the vector's way to the GPU 0.1.
+// ---------------------------------------------------------------------------
+struct RdmList {   // one nonzero column of X for a string
+    uint32_t J;    // string it takes c from
+    int16_t ab;    // column r L + p
+    int16_t sign;
+};
+
+// lists[k][nl]: number operators (J = k), then singles; slot[k][P]: index in
+// the list or -1.
+__global__ void __launch_bounds__(256) k_rdm_lists(uint64_t d, int L, int nel, int S, const str_t* __restrict__ s,
+                                                   const Exc* __restrict__ sub, RdmList* __restrict__ lists,
+                                                   int16_t* __restrict__ slot) {
+    const uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= d) return;
+    const int P = L * L, nl = nel + S - 1;
+    RdmList* o = lists + k * (uint64_t)nl;
+    int16_t* sl = slot + k * (uint64_t)P;
+    for (int p = 0; p < P; ++p) sl[p] = -1;
+    int e = 0;
+    for (str_t t = s[k]; t; t &= t - 1) {
+        const int a = __builtin_ctzll(t);
+        o[e] = RdmList{(uint32_t)k, (int16_t)(a * (L + 1)), 1};
+        sl[a * (L + 1)] = (int16_t)e++;
     }
+    const Exc* x = sub + k * (uint64_t)S;
+    for (int i = 0; i < S; ++i)
+        if (x[i].type == 1) {
+            const int ab = x[i].f * L + x[i].t;
+            o[e] = RdmList{x[i].J, (int16_t)ab, (int16_t)(x[i].sign < 0 ? -1 : 1)};
+            sl[ab] = (int16_t)e++;
+        }
+}
+
+// part[z] = partial C C^T (COLS false: rows of the d x m matrix C) or C^T C
+// (COLS true: columns of the m x d matrix C) over the z-th part of the m
+// dimension; 64 x 64 output blocks, four wavefronts of 2 x 2 MFMA tiles, lower
+// block triangle mirrored.
+constexpr int kMK = 32;
+template <bool COLS>
+__global__ void __launch_bounds__(256) k_string_gram(uint64_t d, uint64_t m, uint64_t per,
+                                                     const double* __restrict__ C, double* __restrict__ part) {
+    __shared__ double As[64][kMK + 1], Bs[64][kMK + 1];
+    if (blockIdx.y > blockIdx.x) return;
+    const uint64_t i0 = (uint64_t)blockIdx.x * 64, j0 = (uint64_t)blockIdx.y * 64;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int r = lane & 15, kq = lane >> 4, wi = (w >> 1) * 32, wj = (w & 1) * 32;
+    const uint64_t k0 = blockIdx.z * per, k1 = k0 + per < m ? k0 + per : m;
+    v4d acc[2][2];
+    for (int a = 0; a < 2; ++a)
+        for (int b = 0; b < 2; ++b) acc[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
+    for (uint64_t kb = k0; kb < k1; kb += kMK) {
+        double a[8], b[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int t = tid + 256 * q;
+            const int x = COLS ? t & 63 : t / kMK, k = COLS ? t >> 6 : t % kMK;
+            const bool in = kb + k < k1;
+            const uint64_t K = kb + k;
+            a[q] = in && i0 + x < d ? C[COLS ? K * d + i0 + x : (i0 + x) * m + K] : 0.0;
+            b[q] = in && j0 + x < d ? C[COLS ? K * d + j0 + x : (j0 + x) * m + K] : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int t = tid + 256 * q;
+            const int x = COLS ? t & 63 : t / kMK, k = COLS ? t >> 6 : t % kMK;
+            As[x][k] = a[q];
+            Bs[x][k] = b[q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < kMK; ks += 4) {
+            double av[2], bv[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                av[t] = As[wi + t * 16 + r][ks + kq];
+                bv[t] = Bs[wj + t * 16 + r][ks + kq];
+            }
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < 2; ++tj)
+                    acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[ti], bv[tj], acc[ti][tj], 0, 0, 0);
+        }
+    }
+    double* o = part + blockIdx.z * d * d;
+#pragma unroll
+    for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const uint64_t i = i0 + wi + ti * 16 + 4 * v + kq, j = j0 + wj + tj * 16 + r;
+                if (i < d && j < d) {
+                    o[i * d + j] = acc[ti][tj][v];
+                    if (blockIdx.y != blockIdx.x) o[j * d + i] = acc[ti][tj][v];
+                }
+            }
+}
+
+// part[z][rp][qs] over the z-th part of the strings: s s' M(J_rp, J_qs); row P
+// of the output is gamma: s M(k, J_qs).  Elements from `first` on.
+__global__ void __launch_bounds__(256) k_same_spin_2rdm(uint64_t d, int P, int nl, uint64_t per, int first,
+                                                        const RdmList* __restrict__ lists,
+                                                        const int16_t* __restrict__ slot, const double* __restrict__ M,
+                                                        double* __restrict__ part) {
+    const int t = first + blockIdx.x * 256 + threadIdx.x;
+    if (t >= (P + 1) * P) return;
+    const int rp = t / P, qs = t - rp * P;
+    const uint64_t k0 = blockIdx.y * per, k1 = k0 + per < d ? k0 + per : d;
+    double acc = 0.0;
+    for (uint64_t k = k0; k < k1; ++k) {
+        const int e2 = slot[k * P + qs], e1 = rp < P ? slot[k * P + rp] : 0;
+        if (e1 < 0 || e2 < 0) continue;
+        const RdmList y = lists[k * nl + e2];
+        const RdmList x = rp < P ? lists[k * nl + e1] : RdmList{(uint32_t)k, 0, 1};
+        const double v = M[(uint64_t)x.J * d + y.J];
+        acc += x.sign == y.sign ? v : -v;
+    }
+    part[(uint64_t)blockIdx.y * (P + 1) * P + t] = acc;
+}
+
+// One alpha string's (or part of its beta range's) opposite-spin block:
+// out[e][qs] = sum_kb X^a_e(ka, kb) X^b_qs(ka, kb), e over the string's list.
+// TB tiles of 16 columns qs, eight wavefronts; TPW output tiles a wavefront.
+constexpr int kAbRows = 32;  // beta strings per LDS stage
+template <int TPW>
+__global__ void __launch_bounds__(512) k_gram_ab(uint64_t db, int P, int nla, int nlb, uint32_t nsplit,
+                                                 const RdmList* __restrict__ la, const RdmList* __restrict__ lb,
+                                                 const double* __restrict__ c, double* __restrict__ part) {
+    extern __shared__ double smem_ab[];
+    const int TA = (nla + 15) / 16, TB = (P + 15) / 16, BS = TB * 16 + 1;
+    double* As = smem_ab;                             // [TA * 16][kAbRows + 1]
+    double* Bs = As + TA * 16 * (kAbRows + 1);        // [kAbRows][BS]
+    const uint64_t ka = blockIdx.x / nsplit;
+    const uint32_t sp = blockIdx.x - (uint32_t)(ka * nsplit);
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int r = lane & 15, kq = lane >> 4, ntiles = TA * TB;
+    const uint64_t steps = (db + kAbRows - 1) / kAbRows;
+    const uint64_t s0 = steps * sp / nsplit, s1 = steps * (sp + 1) / nsplit;
+    v4d acc[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) acc[t] = v4d{0.0, 0.0, 0.0, 0.0};
+    const RdmList* l = la + ka * (uint64_t)nla;
+    const double* row = c + ka * db;
+    for (uint64_t s = s0; s < s1; ++s) {
+        const uint64_t kb0 = s * kAbRows;
+        __syncthreads();  // the last stage has been read
+        for (int i = tid; i < kAbRows * BS; i += 512) Bs[i] = 0.0;
+        for (int i = tid; i < TA * 16 * kAbRows; i += 512) {
+            const int e = i / kAbRows, k = i - e * kAbRows;
+            double v = 0.0;
+            if (e < nla && kb0 + k < db) {
+                const RdmList x = l[e];
+                v = c[(uint64_t)x.J * db + kb0 + k];
+                if (x.sign < 0) v = -v;
+            }
+            As[e * (kAbRows + 1) + k] = v;
+        }
+        __syncthreads();
+        for (int i = tid; i < kAbRows * nlb; i += 512) {
+            const int k = i / nlb;
+            if (kb0 + k >= db) break;
+            const RdmList x = lb[(kb0 + k) * nlb + (i - k * nlb)];
+            const double v = row[x.J];
+            Bs[k * BS + x.ab] = x.sign < 0 ? -v : v;
+        }
+        __syncthreads();
+#pragma unroll 2
+        for (int ks = 0; ks < kAbRows; ks += 4) {
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) {
+                const int tile = w + 8 * t;
+                if (tile < ntiles) {
+                    const int ti = tile / TB, tj = tile - ti * TB;
+                    const double av = As[(ti * 16 + r) * (kAbRows + 1) + ks + kq];
+                    const double bv = Bs[(ks + kq) * BS + tj * 16 + r];
+                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[t], 0, 0, 0);
+                }
+            }
+        }
+    }
+    double* o = part + ((uint64_t)blockIdx.x * nla) * P;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+        const int tile = w + 8 * t;
+        if (tile < ntiles) {
+            const int ti = tile / TB, tj = tile - ti * TB;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int e = ti * 16 + 4 * v + kq, q = tj * 16 + r;
+                if (e < nla && q < P) o[(uint64_t)e * P + q] = acc[t][v];
+            }
+        }
+    }
+}
+
+// part[z][rp][qs] = the blocks of the z-th part of the alpha strings, in order.
+__global__ void __launch_bounds__(256) k_sum_ab(uint64_t da, int P, int nla, uint32_t nsplit, uint64_t per,
+                                                const int16_t* __restrict__ slot, const double* __restrict__ blocks,
+                                                double* __restrict__ part) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= P * P) return;
+    const int rp = t / P, qs = t - rp * P;
+    const uint64_t k0 = blockIdx.y * per, k1 = k0 + per < da ? k0 + per : da;
+    double acc = 0.0;
+    for (uint64_t k = k0; k < k1; ++k) {
+        const int e = slot[k * P + rp];
+        if (e < 0) continue;
+        for (uint32_t s = 0; s < nsplit; ++s) acc += blocks[((k * nsplit + s) * nla + e) * P + qs];
+    }
+    part[(uint64_t)blockIdx.y * P * P + t] = acc;
+}
+
+struct RdmSide {
+    DBuf<RdmList> lists;
+    DBuf<int16_t> slot;
+    int nl = 0;
+};
+
+static void make_side(RdmSide& s, uint64_t d, int L, int nel, int S, const str_t* str, const Exc* sub,
+                      hipStream_t stream) {
+    s.nl = nel + S - 1;
+    s.lists.alloc(std::max<uint64_t>(1, d * (uint64_t)s.nl));
+    s.slot.alloc(d * (uint64_t)L * L);
+    k_rdm_lists<<<(unsigned)((d + 255) / 256), 256, 0, stream>>>(d, L, nel, S, str, sub, s.lists.p, s.slot.p);
+    CF_HIP(hipGetLastError());
+}
+
+// One-spin matrix M = C C^T or C^T C, then that spin's Gram block (with `two`)
+// and, in the last row, gamma into out[(P + 1) P].
+static void same_spin(bool cols, uint64_t d, uint64_t m, int P, const RdmSide& s, const double* c, bool two, double* out,
+                      hipStream_t stream) {
+    const unsigned nb = (unsigned)((d + 63) / 64);
+    // parts of the sum that fill the GPU, of at least 64 terms, within 1 GiB
+    uint64_t z = std::max<uint64_t>(1, 1024 / ((uint64_t)nb * (nb + 1) / 2));
+    z = std::min<uint64_t>({z, (m + 63) / 64, std::max<uint64_t>(1, (1ull << 27) / (d * d))});
+    const uint64_t per = ((m + z - 1) / z + kMK - 1) / kMK * kMK;
+    DBuf<double> parts(z * d * d), M(z > 1 ? d * d : 0);
+    const dim3 grid(nb, nb, (unsigned)z);
+    if (cols) k_string_gram<true><<<grid, 256, 0, stream>>>(d, m, per, c, parts.p);
+    else k_string_gram<false><<<grid, 256, 0, stream>>>(d, m, per, c, parts.p);
+    CF_HIP(hipGetLastError());
+    if (z > 1) {
+        k_sum_chunks<<<(unsigned)((d * d + 255) / 256), 256, 0, stream>>>((int)z, d * d, parts.p, M.p);
+        CF_HIP(hipGetLastError());
+    }
+    const uint64_t len = (uint64_t)(P + 1) * P;
+    const uint64_t y = std::max<uint64_t>(1, std::min<uint64_t>(32, d / 8)), yper = (d + y - 1) / y;
+    const uint64_t first = two ? 0 : (uint64_t)P * P;
+    DBuf<double> sums(y * len);
+    k_same_spin_2rdm<<<dim3((unsigned)((len - first + 255) / 256), (unsigned)y), 256, 0, stream>>>(
+        d, P, s.nl, yper, (int)first, s.lists.p, s.slot.p, z > 1 ? M.p : parts.p, sums.p);
+    CF_HIP(hipGetLastError());
+    // (without `two` the sums of the rows before gamma are of unused memory and not read)
+    k_sum_chunks<<<(unsigned)((len + 255) / 256), 256, 0, stream>>>((int)y, len, sums.p, out);
+    CF_HIP(hipGetLastError());
+}
+
+static void rdm_fci(hipStream_t stream, int L, int na, int nb, uint64_t da, uint64_t db, const str_t* sa, const str_t* sb,
+                    const Exc* suba, const Exc* subb, int Sa, int Sb, const double* c, double* gamma, double* Gamma) {
+    const int P = L * L;
+    const uint64_t PP = (uint64_t)P * P, len = PP + P;
+    RdmSide A, Bown;
+    make_side(A, da, L, na, Sa, sa, suba, stream);
+    const bool same = sa == sb;
+    if (!same) make_side(Bown, db, L, nb, Sb, sb, subb, stream);
+    const RdmSide& B = same ? A : Bown;
+    DBuf<double> G(2 * len + PP);  // aa + gamma_a, bb + gamma_b, ab
+    same_spin(false, da, db, P, A, c, Gamma != nullptr, G.p, stream);
+    same_spin(true, db, da, P, B, c, Gamma != nullptr, G.p + len, stream);
+    if (Gamma) {
+        double* gab = G.p + 2 * len;
+        if (A.nl == 0 || B.nl == 0) {
+            k_zero<<<(unsigned)((PP + 255) / 256), 256, 0, stream>>>(PP, gab);
+            CF_HIP(hipGetLastError());
+        } else {
+            const uint64_t steps = (db + kAbRows - 1) / kAbRows;
+            const uint32_t nsplit = (uint32_t)std::min<uint64_t>(steps, std::max<uint64_t>(1, 1024 / da));
+            DBuf<double> blocks(da * nsplit * (uint64_t)A.nl * P);
+            const int TA = (A.nl + 15) / 16, TB = (P + 15) / 16, tpw = (TA * TB + 7) / 8;
+            const size_t lds = (size_t)(TA * 16 * (kAbRows + 1) + kAbRows * (TB * 16 + 1)) * sizeof(double);
+            const unsigned grid = (unsigned)(da * nsplit);
+#define CF_AB(T)                                                                                                \
+    do {                                                                                                        \
+        if (lds > 64 * 1024)                                                                                    \
+            CF_HIP(hipFuncSetAttribute((const void*)k_gram_ab<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+        k_gram_ab<T><<<grid, 512, lds, stream>>>(db, P, A.nl, B.nl, nsplit, A.lists.p, B.lists.p, c, blocks.p);  \
+    } while (0)
+            if (tpw <= 1) CF_AB(1);
+            else if (tpw <= 3) CF_AB(3);
+            else if (tpw <= 6) CF_AB(6);
+            else CF_AB(10);
+#undef CF_AB
+            CF_HIP(hipGetLastError());
+            const uint64_t y = std::max<uint64_t>(1, std::min<uint64_t>(32, da / 8)), yper = (da + y - 1) / y;
+            DBuf<double> sums(y * PP);
+            k_sum_ab<<<dim3((unsigned)((PP + 255) / 256), (unsigned)y), 256, 0, stream>>>(da, P, A.nl, nsplit, yper,
+                                                                                     A.slot.p, blocks.p, sums.p);
+            CF_HIP(hipGetLastError());
+            k_sum_chunks<<<(unsigned)((PP + 255) / 256), 256, 0, stream>>>((int)y, PP, sums.p, gab);
+            CF_HIP(hipGetLastError());
+        }
+    }
+    std::vector<double> h(2 * len + PP);
+    CF_HIP(hipMemcpyAsync(h.data(), G.p, (Gamma ? 2 * len + PP : 2 * len) * sizeof(double), hipMemcpyDeviceToHost, stream));
+    CF_HIP(hipStreamSynchronize(stream));
+    for (int s = 0; s < 2; ++s) std::copy_n(h.data() + s * len + PP, P, gamma + s * P);
+    if (!Gamma) return;
+    const double* blocks3[3] = {h.data(), h.data() + 2 * len, h.data() + len};
+    unpack_gram(L, blocks3, gamma, Gamma);
 }
 
 void rdm_dense(hipStream_t stream, int kind, int L, int nup, int ndown, uint64_t da, uint64_t db, const str_t* sa,
                const str_t* sb, const Exc* suba, const Exc* subb, int Sa, int Sb, const uint64_t* binom,
                const double* c_host, uint64_t n, double* gamma, double* Gamma) {
-    (void)nup;
-    (void)ndown;
     const int P = L * L;
     DBuf<double> c(n);
     CF_HIP(hipMemcpyAsync(c.p, c_host, n * sizeof(double), hipMemcpyHostToDevice, stream));
     std::vector<double> g(2 * (size_t)P, 0.0);
     if (kind == 1) {  // DOCI
-        uint64_t nchunk = (n + 2047) / 2048;
-        if (nchunk > 1024) nchunk = 1024;
+        // 16 rows a workgroup while that fills the GPU: each thread's bin is a
+        // serial loop over them (252 rows in one workgroup took 151 us)
+        uint64_t nchunk = (n + 15) / 16;
+        if (nchunk > 512) nchunk = 512;
         if (nchunk < 1) nchunk = 1;
         const uint64_t rows = (n + nchunk - 1) / nchunk;
         const uint64_t len = 2 * (uint64_t)P + L;
@@ -350,7 +697,11 @@ void rdm_dense(hipStream_t stream, int kind, int L, int nup, int ndown, uint64_t
         }
         return;
     }
-    // FCI
+    // FCI: one-spin matrices where they are small (2 GiB at most), else X in memory
+    if (L <= 16 && da <= 16384 && db <= 16384) {
+        rdm_fci(stream, L, nup, ndown, da, db, sa, sb, suba, subb, Sa, Sb, c.p, gamma, Gamma);
+        return;
+    }
     DBuf<double> Xa(n * (uint64_t)P), Xb(n * (uint64_t)P);
     CF_HIP(hipMemsetAsync(Xa.p, 0, Xa.bytes(), stream));
     CF_HIP(hipMemsetAsync(Xb.p, 0, Xb.bytes(), stream));
