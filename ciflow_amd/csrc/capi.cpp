@@ -797,6 +797,10 @@ struct DeviceBackend : KrylovBackend {
     // alpha_j v_j + beta_{j-1} v_{j-1} first and then take one full pass, which
     // halves the basis traffic.  alpha_j = (v_j . w) + correction of the pass.
     void orth_deferred(int j) override {
+        if (n <= kStepMaxN && !first_ && j >= 1 && j < 64) {
+            launch_small_step(n, j, Vb.p, w.p, c2.p, scal.p, v(j + 1), dalpha.p, dbeta.p, c->stream);
+            return;
+        }
         if (fused && j + 1 <= 64) {
             // five launches: product, three-term update (or first pass), product,
             // update + |w|^2 parts, normalisation; no separate reductions

@@ -244,6 +244,11 @@ void launch_multi_axpy_r(uint64_t n, int k, int nblocks, const double* partial, 
                          double* c_out, double* pnorm, hipStream_t stream, const double* skip_before = nullptr,
                          const double* skip_after = nullptr, double eta = 0.0);
 // finish_step with |w|^2 = the sum of the fused_axpy_blocks(n) entries of pnorm
+// Step j >= 1 of a small space after its product w = H v_j: alpha_j, the next
+// vector and beta_j in two launches (c: 64 doubles, scal: 2 doubles of scratch).
+constexpr uint64_t kStepMaxN = 16384;
+void launch_small_step(uint64_t n, int j, const double* Vb, const double* w, double* c, double* scal, double* vnext,
+                       double* alpha, double* beta, hipStream_t stream);
 void launch_finish_step_r(uint64_t n, int j, const double* c1, const double* c2, const double* pnorm,
                           const double* w, double* vnext, double* alpha, double* beta, hipStream_t stream);
 void launch_rotate_basis(uint64_t n, int m, int k, double* Vb, const double* Y, hipStream_t stream);
