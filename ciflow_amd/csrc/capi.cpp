@@ -2057,6 +2057,8 @@ void sigma_apply(cf_sigma* S, int prec, const double* x, double* y) {
         launch_to_f32(sp->n, x, S->x32.p, c->stream);
         if (S->shape.kernel != 3 || !launch_sigma_ab3<float>(S->args, sp->ham->ndown, S->x32.p, y, c->stream))
             launch_sigma_ab2<float>(S->args, S->shape, S->x32.p, y, c->stream);
+    } else if (S->shape.kernel == 3 && S->args.sym) {
+        launch_sigma_mfma(S->args, x, y, c->stream);
     } else {
         if (S->shape.kernel != 3 || !launch_sigma_ab3<double>(S->args, sp->ham->ndown, x, y, c->stream))
             launch_sigma_ab2<double>(S->args, S->shape, x, y, c->stream);
@@ -2144,6 +2146,16 @@ int cf_sigma_create(cf_space* sp, int prec, cf_sigma** out) {
         launch_sigma_tables<float>(a, S->vpair32.p, S->vself32.p, c->stream);
         a.vpair32 = S->vpair32.p;
         a.vself32 = S->vself32.p;
+    }
+    if (sigma_mfma_fits(a)) {
+        DBuf<int> sym(1);
+        launch_v_symmetric(a.L, a.V, sym.p, c->stream);
+        S->gat.alloc(sigma_mfma_slots(a));
+        S->gst.alloc(kSigmaStarts);
+        launch_mfma_gather(a, S->gat.p, S->gst.p, c->stream);
+        a.gat = S->gat.p;
+        a.gst = S->gst.p;
+        copy_sync(&a.sym, sym.p, sizeof(int), hipMemcpyDeviceToHost, c->stream);
     }
     CF_HIP(hipStreamSynchronize(c->stream));
     *out = S.release();

@@ -178,6 +178,8 @@ struct cf_sigma {
     SigmaArgs args;
     DBuf<double> vpair64, vself64;  // slice tables of the prefetching alpha-beta kernel
     DBuf<float> vpair32, vself32;
+    DBuf<uint32_t> gat;  // beta actions by column, matrix-product kernel
+    DBuf<uint32_t> gst;
     SigmaShape shape;
     uint64_t version = 0;  // space Hamiltonian version the tables were made for
     // determinant-list spaces (CI_Big): the product on the fly from the

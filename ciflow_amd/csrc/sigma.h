@@ -21,6 +21,11 @@ struct SigmaArgs {
     const double* vself64 = nullptr;
     const float* vpair32 = nullptr;
     const float* vself32 = nullptr;
+    // matrix-product kernel (sigma_mfma.hip): V symmetric in q <-> s, and the
+    // beta actions sorted by pair column
+    int sym = 0;
+    const uint32_t* gat = nullptr;
+    const uint32_t* gst = nullptr;
 };
 
 // Alpha-beta kernel choice: 1 = stage the V slice and C row per alpha action
@@ -70,6 +75,18 @@ bool sigma_ab3_batch_args(SigmaArgs& a, int nb_electrons, bool f32);
 // shape: any lane's args (the lanes share da, db, L and the list lengths).
 template <typename CT>
 void launch_sigma_ab3_batch(const SigmaArgs& shape, int nb_electrons, const SigmaBatch& sb, int lanes, hipStream_t s);
+// The alpha-beta part as a matrix product on FP64 MFMA, for integrals that are
+// symmetric in q <-> s (a.sym): shapes whose F columns fit in LDS (d_b <= 1,024,
+// at most 40 alpha actions, L <= 16).  Tables gat (sigma_mfma_slots entries) and
+// gst (kSigmaStarts) depend on the strings alone.
+constexpr int kSigmaStarts = 33;
+bool sigma_mfma_fits(const SigmaArgs& a);
+uint64_t sigma_mfma_slots(const SigmaArgs& a);
+void launch_mfma_gather(const SigmaArgs& a, uint32_t* gat, uint32_t* gst, hipStream_t s);
+void launch_v_symmetric(int L, const double* V, int* sym, hipStream_t s);
+void launch_sigma_mfma(const SigmaArgs& a, const double* C, double* sig, hipStream_t s);
+// lanes of the batch with FP64 operands and a.sym (the others do nothing)
+void launch_sigma_mfma_batch(const SigmaArgs& shape, const SigmaBatch& sb, int lanes, hipStream_t s);
 template <typename T>
 void launch_dense_string_ham(uint64_t d, int E, const Exc* full, T* H, hipStream_t s);
 void launch_to_f32(uint64_t n, const double* x, float* y, hipStream_t s);

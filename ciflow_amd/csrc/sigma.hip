@@ -505,6 +505,7 @@ __global__ void __launch_bounds__(NT) k_sigma_ab3(SigmaArgs a0, const CT* __rest
         const BdStep& st = sb.step[lane];
         if (st.mode == BD_IDLE || st.f32 != (S == 4 ? 1 : 0)) return;
         a = sb.args[lane];
+        if (S == 8 && a.sym) return;  // the matrix-product kernel's
         const uint64_t off = ((uint64_t)lane * sb.M + st.m) * sb.n;
         C = S == 4 ? reinterpret_cast<const CT*>(sb.x32 + (uint64_t)lane * sb.n) : reinterpret_cast<const CT*>(sb.V + off);
         sig = sb.S + off;

@@ -104,6 +104,8 @@ struct Batch {
     DBuf<BdOpLane> dop;
     DBuf<SigmaArgs> dargs;
     cf_ctx::DociBlockTables* blk = nullptr;
+    DBuf<uint32_t> gat;  // FCI: beta actions by pair column (strings only, shared by the lanes)
+    DBuf<uint32_t> gst;
     BdView view;
     // page-locked staging
     BdStep* hstep = nullptr;
@@ -196,6 +198,7 @@ void Batch::add(const std::vector<std::pair<int, cf_request>>& in) {
             for (int a = 0; a < L; ++a) uu[i * L2 + a * L + a] = 1.0;
     }
     DBuf<double> dh(k * L2), dV(k * L4), dU(k * L2), oh(k * L2), oV(k * L4), tmp(k * L4);
+    DBuf<int> sym(k);
     CF_HIP(hipMemcpyAsync(dh.p, hh.data(), dh.bytes(), hipMemcpyHostToDevice, st));
     CF_HIP(hipMemcpyAsync(dV.p, vv.data(), dV.bytes(), hipMemcpyHostToDevice, st));
     CF_HIP(hipMemcpyAsync(dU.p, uu.data(), dU.bytes(), hipMemcpyHostToDevice, st));
@@ -294,7 +297,16 @@ void Batch::add(const std::vector<std::pair<int, cf_request>>& in) {
                 a.vself32 = q.vself32.p;
             }
             CF_REQUIRE(sigma_ab3_batch_args(a, ndown, false), "batched sigma: no kernel for this shape");
-            hargs[b] = a;
+            if (sigma_mfma_fits(a)) {
+                if (!gst.p) {
+                    gat.alloc(sigma_mfma_slots(a));
+                    gst.alloc(kSigmaStarts);
+                    launch_mfma_gather(a, gat.p, gst.p, st);
+                }
+                a.gat = gat.p;
+                a.gst = gst.p;
+                launch_v_symmetric(L, a.V, sym.p + i, st);
+            }
         }
         // solver state: the FP32 phase first for FP32 requests
         q.G.assign((size_t)M * M, 0.0);
@@ -312,6 +324,18 @@ void Batch::add(const std::vector<std::pair<int, cf_request>>& in) {
         q.krylov = 8;
         q.start = true;
         q.start_mode = BD_START_SEED;
+    }
+    if (kind == CF_FCI) {
+        std::vector<int> hsym(k, 0);
+        if (gst.p) {
+            CF_HIP(hipMemcpyAsync(hsym.data(), sym.p, k * sizeof(int), hipMemcpyDeviceToHost, st));
+            CF_HIP(hipStreamSynchronize(st));
+        }
+        for (int i = 0; i < k; ++i) {
+            Lane& q = lanes[slot[i]];
+            q.args.sym = hsym[i];
+            hargs[slot[i]] = q.args;
+        }
     }
     CF_HIP(hipMemcpyAsync(dop.p, hop.data(), cap * sizeof(BdOpLane), hipMemcpyHostToDevice, st));
     if (kind == CF_FCI)
@@ -334,10 +358,15 @@ void Batch::product(bool any32, bool any64) {
         sb.n = n;
         sb.M = M;
         const SigmaArgs* shape = nullptr;
+        bool sym = false, asym = false;  // lanes of either FP64 kernel
         for (const Lane& q : lanes)
-            if (q.id >= 0) shape = &q.args;
+            if (q.id >= 0) {
+                shape = &q.args;
+                (q.args.sym ? sym : asym) = true;
+            }
         if (any32) launch_sigma_ab3_batch<float>(*shape, ndown, sb, cap, st);
-        if (any64) launch_sigma_ab3_batch<double>(*shape, ndown, sb, cap, st);
+        if (any64 && sym) launch_sigma_mfma_batch(*shape, sb, cap, st);
+        if (any64 && asym) launch_sigma_ab3_batch<double>(*shape, ndown, sb, cap, st);
     } else {
         DociBatch bt;
         bt.step = dstep.p;

@@ -315,8 +315,10 @@ int cf_sigma_set_threads(cf_sigma* s, int threads);
 /* Alpha-beta kernel (tuning; no reference counterpart): 1 = stage each alpha
  * action's V slice and C row, 2 = per-Hamiltonian slice tables with the next
  * action's slice and row prefetched into registers (shapes it does not cover
- * run kernel 1), 3 (default) = kernel 2 with packed LDS offsets and exact
- * beta-list lengths (shapes without an instance run kernel 2). */
+ * run kernel 1), 3 (default) = in FP64, for V[p][q][r][s] = V[p][s][r][q] (real
+ * orbitals) and up to 1,024 beta strings, a matrix product over the alpha
+ * actions; otherwise kernel 2 with packed LDS offsets and exact beta-list
+ * lengths (shapes without an instance run kernel 2). */
 int cf_sigma_set_kernel(cf_sigma* s, int kernel);
 /* ---- CI_Big (CIMethod.h:176-189, CIMethod.cpp:591-609, 943-1116, 1118-1142):
  *      a determinant-list space (cf_space_create_dets, L <= 32) whose matrix
