@@ -117,80 +117,230 @@ __global__ void __launch_bounds__(256) k_bd_rotate(BdView b) {
     }
 }
 
-// BD_RITZ: x = V y, r = S y - theta x, t = r / (theta - diag) (t = r when
-// shift is 0), parts of |r|^2 and |t|^2.  BD_START_X / BD_START_SEED: t
-// = x or the seeded start vector, parts of |t|^2 (|r|^2 parts zero).
-__global__ void __launch_bounds__(256) k_bd_combine(BdView b) {
+// The passes that make t read the basis once: a thread keeps its element of up
+// to 24 basis vectors in registers (kChunk at a time, C chunks; rows past k
+// repeat row k - 1 with coefficient 0), forms t there and at once the dot
+// products V^T t that the next Gram-Schmidt pass needs.  HBM- and L2-bound: with
+// a pass of its own over V for those dots the vector passes of a step took 242 us
+// for 12 x FCI L=11 (5,5) and 123 us for 12 x DOCI L=19, now 167 and 85.
+// Workgroups of 512, at most 64 a lane: 183 VGPRs hold the 24-vector instance
+// (at the 128 of twice as many wavefronts it spilled 104).
+// The rows' addresses stay in scalar registers: a uniform base per row and a
+// byte offset per lane.
+__device__ __forceinline__ double at(const double* base, uint32_t off) {
+    return *(const double*)((const char*)base + off);
+}
+template <int C>
+__device__ __forceinline__ void load_basis(const double* __restrict__ V, int k, uint64_t n, uint64_t q0, uint32_t off,
+                                           double* v) {
+#pragma unroll
+    for (int i = 0; i < C * kChunk; ++i) v[i] = at(V + ((uint64_t)min(i, k - 1) * n + q0), off);
+}
+
+// One value a lane of eight, summed over the wavefront: halves of the values
+// change hands at distances 32, 16 and 8 (ten shuffles instead of 48).  Lane l
+// returns the sum of value l >> 3.
+__device__ __forceinline__ double wave_sum8(const double* a) {
+    const int l = threadIdx.x & 63;
+    double b[4], c[2];
+    const bool h5 = l & 32, h4 = l & 16, h3 = l & 8;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[j] = (h5 ? a[j + 4] : a[j]) + __shfl_xor(h5 ? a[j] : a[j + 4], 32, 64);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) c[j] = (h4 ? b[j + 2] : b[j]) + __shfl_xor(h4 ? b[j] : b[j + 2], 16, 64);
+    double d = (h3 ? c[1] : c[0]) + __shfl_xor(h3 ? c[0] : c[1], 8, 64);
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+    return d;
+}
+
+constexpr int kFusedThreads = 512;
+struct FusedSums {
+    double dots[kDavMaxBasis][kFusedThreads / 64];
+    double norms[2][kFusedThreads / 64];
+};
+
+// The workgroup's dot partials (into partial[i * Gd + block]) and norm parts.
+template <int C>
+__device__ __forceinline__ void put_sums(FusedSums& f, int k, double* acc, double n0, double n1, int Gd,
+                                         double* partial, double* part0, double* part1) {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const double s = wave_sum8(acc + c * kChunk);
+        if ((l & 7) == 0) f.dots[c * kChunk + (l >> 3)][w] = s;
+    }
+    n0 = wave_sum(n0);
+    n1 = wave_sum(n1);
+    if (l == 0) {
+        f.norms[0][w] = n0;
+        f.norms[1][w] = n1;
+    }
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i < k + 2) {
+        const double* r = i < k ? f.dots[i] : f.norms[i - k];
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < kFusedThreads / 64; ++q) s += r[q];
+        if (i < k) partial[(size_t)i * Gd + blockIdx.x] = s;
+        else if (i == k) part0[blockIdx.x] = s;
+        else if (part1) part1[blockIdx.x] = s;
+    }
+}
+
+// BD_RITZ: x = V y (stored for lanes whose solve goes on in FP64 from it),
+// r = S y - theta x, t = r / (theta - diag) (t = r when shift is 0), parts of
+// |r|^2 and |t|^2, and V^T t.
+template <int C>
+__device__ __forceinline__ void ritz(const BdView& b, int lane, const BdStep& st, const double* ys, FusedSums& f,
+                                     double* P, double* partial) {
+    const uint64_t n = b.n;
+    const int k = st.m;
+    const double theta = st.theta, shift_min = st.shift;
+    const double* V = b.V + (uint64_t)lane * b.M * n;
+    const double* S = b.S + (uint64_t)lane * b.M * n;
+    double* x = st.f32 ? b.x + (uint64_t)lane * n : nullptr;
+    double* t = b.t + (uint64_t)lane * n;
+    const double* diag = b.op[lane].diag;
+    double acc[C * kChunk], nr = 0.0, nt = 0.0;
+#pragma unroll
+    for (int i = 0; i < C * kChunk; ++i) acc[i] = 0.0;
+    for (uint64_t q0 = (uint64_t)blockIdx.x * kFusedThreads; q0 < n; q0 += (uint64_t)b.Gd * kFusedThreads) {
+        const uint32_t left = (uint32_t)min(n - q0, (uint64_t)kFusedThreads);
+        const bool in = threadIdx.x < left;
+        const uint32_t off = min(threadIdx.x, left - 1) * 8u;
+        double v[C * kChunk], a = 0.0, c = 0.0;
+        asm volatile("" ::: "memory");  // the coefficients are read again from LDS, not kept in registers
+        const double dq = at(diag + q0, off);
+        load_basis<C>(V, k, n, q0, off, v);
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            double w[kChunk];
+#pragma unroll
+            for (int i = 0; i < kChunk; ++i) w[i] = at(S + ((uint64_t)min(j * kChunk + i, k - 1) * n + q0), off);
+#pragma unroll
+            for (int i = 0; i < kChunk; ++i) c += ys[j * kChunk + i] * w[i];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < C * kChunk; ++i) a += ys[i] * v[i];
+        const double r = in ? c - theta * a : 0.0;
+        nr += r * r;
+        double tq = r;
+        if (shift_min > 0.0) {
+            double den = theta - dq;
+            if (fabs(den) < shift_min) den = den < 0.0 ? -shift_min : shift_min;
+            tq = r / den;
+        }
+        if (in) {
+            t[q0 + threadIdx.x] = tq;
+            if (x) x[q0 + threadIdx.x] = a;
+        }
+        nt += tq * tq;
+#pragma unroll
+        for (int i = 0; i < C * kChunk; ++i) acc[i] += v[i] * tq;
+    }
+    put_sums<C>(f, k, acc, nr, nt, b.Gd, partial, P + 512, P + 768);
+}
+
+// BD_START_X / BD_START_SEED: t = x or the seeded start vector, parts of
+// |t|^2 (|r|^2 parts zero).
+__global__ void __launch_bounds__(kFusedThreads, 2) k_bd_combine(BdView b) {
     const int lane = blockIdx.y;
     const BdStep& st = b.step[lane];
     const int mode = st.mode;
     if (mode == BD_IDLE) return;
     __shared__ double ys[kDavMaxBasis];
-    __shared__ double red[2][4];
-    const uint64_t n = b.n;
-    const int k = mode == BD_RITZ ? st.m : 0;
-    if (threadIdx.x < kDavMaxBasis) ys[threadIdx.x] = (int)threadIdx.x < k ? st.ys[threadIdx.x] : 0.0;
-    __syncthreads();
-    const double theta = st.theta, shift_min = st.shift;
-    const uint64_t seed = st.seed;
-    const double* V = b.V + (uint64_t)lane * b.M * n;
-    const double* S = b.S + (uint64_t)lane * b.M * n;
-    double* x = b.x + (uint64_t)lane * n;
+    __shared__ FusedSums f;
+    double* P = lane_parts(b, lane);
+    double* partial = b.partial + (size_t)lane * kBdPartial;
+    if (mode == BD_RITZ) {
+        const int k = st.m;
+        if (threadIdx.x < kDavMaxBasis) ys[threadIdx.x] = (int)threadIdx.x < k ? st.ys[threadIdx.x] : 0.0;
+        __syncthreads();
+        if (k <= kChunk) ritz<1>(b, lane, st, ys, f, P, partial);
+        else if (k <= 2 * kChunk) ritz<2>(b, lane, st, ys, f, P, partial);
+        else ritz<3>(b, lane, st, ys, f, P, partial);
+        return;
+    }
+    const uint64_t n = b.n, seed = st.seed;
+    const double* x = b.x + (uint64_t)lane * n;
     double* t = b.t + (uint64_t)lane * n;
-    const double* diag = b.op[lane].diag;
-    double acc = 0.0, acct = 0.0;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += stride) {
-        double tq;
-        if (mode == BD_RITZ) {
-            double a = 0.0, c = 0.0;
-            combine2(V, S, ys, k, n, q, a, c);
-            x[q] = a;
-            const double r = c - theta * a;
-            acc += r * r;
-            tq = r;
-            if (shift_min > 0.0) {
-                double den = theta - diag[q];
-                if (fabs(den) < shift_min) den = den < 0.0 ? -shift_min : shift_min;
-                tq = r / den;
-            }
-        } else {
-            tq = mode == BD_START_X ? x[q] : start_element(seed, q);
-        }
+    double nt = 0.0;
+    for (uint64_t q = (uint64_t)blockIdx.x * kFusedThreads + threadIdx.x; q < n; q += (uint64_t)b.Gd * kFusedThreads) {
+        const double tq = mode == BD_START_X ? x[q] : start_element(seed, q);
         t[q] = tq;
-        acct += tq * tq;
+        nt += tq * tq;
     }
-    acc = wave_sum(acc);
-    acct = wave_sum(acct);
-    if ((threadIdx.x & 63) == 0) {
-        red[0][threadIdx.x >> 6] = acc;
-        red[1][threadIdx.x >> 6] = acct;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double* P = lane_parts(b, lane);
-        P[512 + blockIdx.x] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-        P[768 + blockIdx.x] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
-    }
+    put_sums<0>(f, 0, nullptr, 0.0, nt, b.Gd, partial, P + 512, P + 768);
 }
 
-// Dot products of basis vectors with w, partial[i * Gd + block]: pass 0
-// V[0:m] . t, pass 1 the same after the first Gram-Schmidt pass (skipped
-// when that pass kept more than eta of t), pass 2 V[0:m+1] . S_m.
-__global__ void __launch_bounds__(1024) k_bd_dot(BdView b, int pass, double eta2) {
+// First Gram-Schmidt pass: t -= V c (c from k_bd_combine's dot partials),
+// parts of |t|^2 after, and V^T t of the result for a second pass.
+template <int C>
+__device__ __forceinline__ void orth1(const BdView& b, int lane, int k, const double* cs, FusedSums& f, double* P,
+                                      double* partial) {
+    const uint64_t n = b.n;
+    const double* V = b.V + (uint64_t)lane * b.M * n;
+    double* t = b.t + (uint64_t)lane * n;
+    double acc[C * kChunk], nt = 0.0;
+#pragma unroll
+    for (int i = 0; i < C * kChunk; ++i) acc[i] = 0.0;
+    for (uint64_t q0 = (uint64_t)blockIdx.x * kFusedThreads; q0 < n; q0 += (uint64_t)b.Gd * kFusedThreads) {
+        const uint32_t left = (uint32_t)min(n - q0, (uint64_t)kFusedThreads);
+        const bool in = threadIdx.x < left;
+        const uint32_t off = min(threadIdx.x, left - 1) * 8u;
+        double v[C * kChunk], s = 0.0;
+        asm volatile("" ::: "memory");
+        const double tq = at(t + q0, off);
+        load_basis<C>(V, k, n, q0, off, v);
+#pragma unroll
+        for (int i = 0; i < C * kChunk; ++i) s += cs[i] * v[i];
+        const double wn = in ? tq - s : 0.0;
+        if (in) t[q0 + threadIdx.x] = wn;
+        nt += wn * wn;
+#pragma unroll
+        for (int i = 0; i < C * kChunk; ++i) acc[i] += v[i] * wn;
+    }
+    put_sums<C>(f, k, acc, nt, 0.0, b.Gd, partial, P, nullptr);
+}
+
+__global__ void __launch_bounds__(kFusedThreads, 4) k_bd_orth1(BdView b) {
+    const int lane = blockIdx.y;
+    const BdStep& st = b.step[lane];
+    if (st.mode == BD_IDLE) return;
+    __shared__ double cs[64];
+    __shared__ FusedSums f;
+    double* P = lane_parts(b, lane);
+    double* partial = b.partial + (size_t)lane * kBdPartial;
+    const int k = st.m;
+    if (k == 0) {  // a start vector: nothing to project out
+        if (threadIdx.x == 0) P[blockIdx.x] = P[768 + blockIdx.x];
+        return;
+    }
+    if (threadIdx.x < 64) cs[threadIdx.x] = 0.0;
+    __syncthreads();
+    if (threadIdx.x < 256) reduce_coeffs(k, b.Gd, partial, cs);
+    __syncthreads();
+    double* next = partial + kBdPartial / 2;
+    if (k <= kChunk) orth1<1>(b, lane, k, cs, f, P, next);
+    else if (k <= 2 * kChunk) orth1<2>(b, lane, k, cs, f, P, next);
+    else orth1<3>(b, lane, k, cs, f, P, next);
+}
+
+// V[0:m+1] . S_m, partial[i * Gd + block].
+__global__ void __launch_bounds__(1024) k_bd_dot(BdView b) {
     const int lane = blockIdx.z;
     const BdStep& st = b.step[lane];
     if (st.mode == BD_IDLE) return;
-    const int m = st.m;
-    const int k = pass == 2 ? m + 1 : m;
+    const int m = st.m, k = m + 1;
     const int i0 = blockIdx.y * kChunk;
     if (i0 >= k) return;
     __shared__ double red[kChunk][16];
     const uint64_t n = b.n;
-    const double* P = lane_parts(b, lane);
-    if (pass == 1 && dgks_skip(P + 768, P, b.Ga, eta2)) return;
     const double* Vb = b.V + (uint64_t)lane * b.M * n;
-    const double* w = pass == 2 ? b.S + ((uint64_t)lane * b.M + m) * n : b.t + (uint64_t)lane * n;
+    const double* w = b.S + ((uint64_t)lane * b.M + m) * n;
     double* partial = b.partial + (size_t)lane * kBdPartial;
     double acc[kChunk];
 #pragma unroll
@@ -199,15 +349,11 @@ __global__ void __launch_bounds__(1024) k_bd_dot(BdView b, int pass, double eta2
     for (uint64_t q = (uint64_t)blockIdx.x * 1024 + threadIdx.x; q < n; q += stride) {
         const double wq = w[q];
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j)
-            if (i0 + j < k) acc[j] += Vb[(uint64_t)(i0 + j) * n + q] * wq;
+        for (int j = 0; j < kChunk; ++j) acc[j] += Vb[(uint64_t)min(i0 + j, m) * n + q] * wq;
     }
     const int l = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j < kChunk; ++j) {
-        const double s = wave_sum(acc[j]);
-        if (l == 0) red[j][wid] = s;
-    }
+    const double sum = wave_sum8(acc);
+    if ((l & 7) == 0) red[l >> 3][wid] = sum;
     __syncthreads();
     if (threadIdx.x < kChunk && i0 + (int)threadIdx.x < k) {
         double s = 0.0;
@@ -216,9 +362,9 @@ __global__ void __launch_bounds__(1024) k_bd_dot(BdView b, int pass, double eta2
     }
 }
 
-// t -= V[0:m] c (c from the pass's dot partials) and parts of |t|^2 after:
-// pass 0 into pnorm, pass 1 (the gated second pass) into pnorm2.
-__global__ void __launch_bounds__(256) k_bd_axpy(BdView b, int pass, double eta2) {
+// Second Gram-Schmidt pass, unless the first one kept more than eta of t:
+// t -= V c (c from k_bd_orth1's dot partials) and parts of |t|^2 after.
+__global__ void __launch_bounds__(256) k_bd_orth2(BdView b, double eta2) {
     const int lane = blockIdx.y;
     const BdStep& st = b.step[lane];
     if (st.mode == BD_IDLE) return;
@@ -226,9 +372,9 @@ __global__ void __launch_bounds__(256) k_bd_axpy(BdView b, int pass, double eta2
     __shared__ double red[4];
     const uint64_t n = b.n;
     double* P = lane_parts(b, lane);
-    if (pass == 1 && dgks_skip(P + 768, P, b.Ga, eta2)) return;
+    if (dgks_skip(P + 768, P, b.Gd, eta2)) return;
     const int k = st.m;
-    reduce_coeffs(k, b.Gd, b.partial + (size_t)lane * kBdPartial, cs);
+    reduce_coeffs(k, b.Gd, b.partial + (size_t)lane * kBdPartial + kBdPartial / 2, cs);
     __syncthreads();
     const double* Vb = b.V + (uint64_t)lane * b.M * n;
     double* w = b.t + (uint64_t)lane * n;
@@ -243,7 +389,7 @@ __global__ void __launch_bounds__(256) k_bd_axpy(BdView b, int pass, double eta2
     nrm = wave_sum(nrm);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = nrm;
     __syncthreads();
-    if (threadIdx.x == 0) P[(pass ? 256 : 0) + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (threadIdx.x == 0) P[256 + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // v_m = t / |t| (|t|^2 from the last pass that ran), its FP32 copy for FP32
@@ -255,10 +401,10 @@ __global__ void __launch_bounds__(256) k_bd_scale(BdView b, double eta2) {
     __shared__ double red[2][4];
     const uint64_t n = b.n;
     const double* P = lane_parts(b, lane);
-    const int np = b.Ga;
-    const double* pnorm = dgks_skip(P + 768, P, np, eta2) ? P : P + 256;
-    double a = (int)threadIdx.x < np ? pnorm[threadIdx.x] : 0.0;
-    double r = (int)threadIdx.x < np ? P[512 + threadIdx.x] : 0.0;
+    const bool one = dgks_skip(P + 768, P, b.Gd, eta2);
+    const double* pnorm = one ? P : P + 256;
+    double a = (int)threadIdx.x < (one ? b.Gd : b.Ga) ? pnorm[threadIdx.x] : 0.0;
+    double r = (int)threadIdx.x < b.Gd ? P[512 + threadIdx.x] : 0.0;
     a = wave_sum(a);
     r = wave_sum(r);
     if ((threadIdx.x & 63) == 0) {
@@ -456,12 +602,10 @@ void bd_form_vectors(const BdView& b, int lanes, bool any_restart, hipStream_t s
         if (tiles > 0xffffffffull) throw Error(ERR_UNSUPPORTED, "batched Davidson: n too large");
         k_bd_rotate<<<dim3((unsigned)tiles, lanes, 2), 256, 0, s>>>(b);
     }
-    const dim3 ga((unsigned)b.Ga, lanes), gd((unsigned)b.Gd, (kDavMaxBasis + kChunk - 1) / kChunk, lanes);
-    k_bd_combine<<<ga, 256, 0, s>>>(b);
-    k_bd_dot<<<gd, 1024, 0, s>>>(b, 0, kEta2);
-    k_bd_axpy<<<ga, 256, 0, s>>>(b, 0, kEta2);
-    k_bd_dot<<<gd, 1024, 0, s>>>(b, 1, kEta2);
-    k_bd_axpy<<<ga, 256, 0, s>>>(b, 1, kEta2);
+    const dim3 ga((unsigned)b.Ga, lanes), gd((unsigned)b.Gd, lanes);
+    k_bd_combine<<<gd, kFusedThreads, 0, s>>>(b);
+    k_bd_orth1<<<gd, kFusedThreads, 0, s>>>(b);
+    k_bd_orth2<<<ga, 256, 0, s>>>(b, kEta2);
     k_bd_scale<<<ga, 256, 0, s>>>(b, kEta2);
     CF_HIP(hipGetLastError());
 }
@@ -469,7 +613,7 @@ void bd_form_vectors(const BdView& b, int lanes, bool any_restart, hipStream_t s
 void bd_new_column(const BdView& b, int lanes, hipStream_t s) {
     check_view(b, lanes);
     const dim3 gd((unsigned)b.Gd, (kDavMaxBasis + kChunk - 1) / kChunk, lanes);
-    k_bd_dot<<<gd, 1024, 0, s>>>(b, 2, kEta2);
+    k_bd_dot<<<gd, 1024, 0, s>>>(b);
     k_bd_reduce<<<dim3(kDavMaxBasis, lanes), 64, 0, s>>>(b);
     CF_HIP(hipGetLastError());
 }

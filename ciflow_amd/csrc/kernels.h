@@ -260,7 +260,8 @@ void launch_copy(uint64_t n, const double* src, double* dst, hipStream_t stream)
 // advanced in lock step, one launch per step for all of them.
 // ---------------------------------------------------------------------------
 constexpr int kBdMaxLanes = 32;
-constexpr int kBdPartial = 64 * 64;  // per lane: dot partials, rows x fused_dot_blocks(n)
+constexpr int kBdPartial = 64 * 64;  // per lane: two sets of dot partials, rows x fused_dot_blocks(n)
+static_assert(2 * kDavMaxBasis * 64 <= kBdPartial, "both Gram-Schmidt passes' partials");
 constexpr int kBdParts = 5 * 256;    // per lane: pnorm, pnorm2, rparts, tparts, r1parts
 enum BdMode : int { BD_IDLE = 0, BD_RITZ = 1, BD_START_X = 2, BD_START_SEED = 3 };
 // One lane's part of an iteration, written by the host before each one.
@@ -292,12 +293,12 @@ struct BdView {
     int Ga = 0, Gd = 0;  // fused_axpy_blocks(n), fused_dot_blocks(n)
     double* V = nullptr;  // [lanes][M][n]
     double* S = nullptr;  // [lanes][M][n] images H V
-    double* x = nullptr;  // [lanes][n] Ritz vector
+    double* x = nullptr;  // [lanes][n] Ritz vector of an FP32-operand phase
     double* t = nullptr;  // correction / new vector before normalisation
     float* x32 = nullptr;  // [lanes][n] FP32 copy of the new vector (or null)
     double* partial = nullptr;  // [lanes][kBdPartial]
     double* parts = nullptr;    // [lanes][kBdParts]
-    double* dg = nullptr;       // [lanes][64]: rows 0..m dots V^T S_m, 62 |r|^2, 63 |t|^2
+    double* dg = nullptr;       // [lanes][64], page-locked host memory: rows 0..m dots V^T S_m, 62 |r|^2, 63 |t|^2
     double* Y = nullptr;        // [lanes][kDavMaxBasis^2] restart rotations
     const BdStep* step = nullptr;  // [lanes]
     const BdOpLane* op = nullptr;  // [lanes]

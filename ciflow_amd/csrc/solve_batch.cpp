@@ -98,7 +98,7 @@ struct Batch {
     std::vector<Lane> lanes;  // cap slots
     std::vector<BdOpLane> hop;
     std::vector<SigmaArgs> hargs;
-    DBuf<double> V, S, x, t, partial, parts, dg, Y;
+    DBuf<double> V, S, x, t, partial, parts, Y;
     DBuf<float> x32;
     DBuf<BdStep> dstep;
     DBuf<BdOpLane> dop;
@@ -142,7 +142,6 @@ void Batch::alloc() {
     if (kind == CF_FCI) x32.alloc(Bn);
     partial.alloc((size_t)cap * kBdPartial);
     parts.alloc((size_t)cap * kBdParts);
-    dg.alloc((size_t)cap * 64);
     Y.alloc((size_t)cap * kDavMaxBasis * kDavMaxBasis);
     dstep.alloc(cap);
     dop.alloc(cap);
@@ -158,7 +157,6 @@ void Batch::alloc() {
     view.x32 = x32.p;
     view.partial = partial.p;
     view.parts = parts.p;
-    view.dg = dg.p;
     view.Y = Y.p;
     view.step = dstep.p;
     view.op = dop.p;
@@ -169,6 +167,7 @@ void Batch::alloc() {
     hstep = (BdStep*)p;
     p += cap * sizeof(BdStep);
     hdg = (double*)p;
+    view.dg = hdg;  // a few numbers a lane: written by the kernels, no copy to wait for
     p += cap * 64 * sizeof(double);
     hr1 = (double*)p;
     p += cap * 256 * sizeof(double);
@@ -519,7 +518,6 @@ void Batch::run() {
         bd_form_vectors(view, cap, any_restart, st);
         product(any32, any64);
         bd_new_column(view, cap, st);
-        CF_HIP(hipMemcpyAsync(hdg, dg.p, (size_t)cap * 64 * sizeof(double), hipMemcpyDeviceToHost, st));
         CF_HIP(hipStreamSynchronize(st));
         std::vector<int> temple;
         for (int b = 0; b < cap; ++b) {
