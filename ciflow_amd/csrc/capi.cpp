@@ -146,7 +146,7 @@ struct cf_crs {
     // DOCI block tables (kernel 6)
     DBuf<DociBlock> dblk;
     DBuf<uint16_t> drank_lo, dlo_of;
-    DBuf<uint32_t> dlo_off;
+    DBuf<uint32_t> dlo_off, dhops;
     DociBlockArgs bargs;
     bool blk_ready = false;
     // sliced copy of the CRS rows (kernel 7): 64-row chunks, quad offsets per
@@ -272,6 +272,10 @@ void make_doci_block_tables(cf_ctx* c, int L, int np, int w, cf_ctx::DociBlockTa
     b.binom = c->binom.p;
     b.diag = nullptr;
     b.zero = 0.0;
+    T.hops.alloc(doci_hop_words(w));
+    b.hops = T.hops.p;
+    launch_doci_hop_table(b, T.hops.p, c->stream);
+    CF_HIP(hipStreamSynchronize(c->stream));
 }
 }  // namespace cf
 
@@ -429,6 +433,7 @@ void make_doci_blocks(cf_crs* m, int w) {
     m->drank_lo = std::move(T.rank_lo);
     m->dlo_of = std::move(T.lo_of);
     m->dlo_off = std::move(T.lo_off);
+    m->dhops = std::move(T.hops);
     m->bargs = T.args;
     m->bargs.n = m->n;
     m->bargs.diag = sp->diag.p;

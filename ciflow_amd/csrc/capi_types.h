@@ -48,7 +48,7 @@ struct cf_ctx {
     struct DociBlockTables {
         cf::DBuf<cf::DociBlock> blocks;
         cf::DBuf<uint16_t> rank_lo, lo_of;
-        cf::DBuf<uint32_t> lo_off;
+        cf::DBuf<uint32_t> lo_off, hops;
         cf::DociBlockArgs args;
     };
     std::map<std::pair<int, int>, DociBlockTables> doci_blk;

@@ -48,10 +48,14 @@ struct DociBlockArgs {
     const uint16_t* rank_lo = nullptr;  // [2^w]: rank of a low pattern among those of its popcount
     const uint16_t* lo_of = nullptr;    // [2^w]: low patterns by popcount, rank order
     const uint32_t* lo_off = nullptr;   // [w + 2]: start of each popcount in lo_of
+    const uint32_t* hops = nullptr;     // [doci_hop_words(w)]: LDS offsets of every low pattern's hops
     const uint64_t* binom = nullptr;
     const double* diag = nullptr;
     double zero = 0.0;
 };
+// Words of the hop table, and the table from the pattern tables of a.
+size_t doci_hop_words(int w);
+void launch_doci_hop_table(const DociBlockArgs& a, uint32_t* words, hipStream_t s);
 // The lanes of a batched Davidson product (block-staged kernel): lane l
 // (grid row l) takes its pair table and diagonal from op[l] and multiplies
 // the new vector of its step, V_m, into S_m; lanes whose step is idle or of
