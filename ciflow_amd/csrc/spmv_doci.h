@@ -31,7 +31,7 @@ DociShape doci_default_shape(uint64_t n);
 // and L - w high ones; the rows whose strings share the high part `hi` (and so
 // hold c = np - popcount(hi) low pairs) are one contiguous rank range,
 // base(hi, c) + rank_lo(lo), a "block".  A workgroup owns a block and stages
-// in LDS its own x block and, one at a time, the x blocks that the hops
+// in LDS its own x block and, a pair at a time, the x blocks that the hops
 // crossing the split reach; hops inside the high part read the neighbour
 // block with coalesced loads.
 struct DociBlock {
@@ -68,7 +68,7 @@ struct DociBatch {
     uint64_t n = 0;
     int M = 0;
 };
-// Largest low part: C(12, 6) = 924 rows per block, 4 per thread of 256.
+// Largest low part: C(12, 6) = 924 rows per block, 2 per thread of 512.
 constexpr int kDociMaxW = 12;
 // Low orbitals for L orbitals (the block shape the kernel is run with by default).
 int doci_block_w(int L);
