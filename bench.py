@@ -6,7 +6,7 @@ uniform in [8, 11], half filling, integrals from seed 1000+k rotated by
 U = exp(K), K antisymmetric with N(0, 0.05^2) entries.  Each request's
 precision is CF_PREC_AUTO (--served-precision): FP32 values + FP64 polish
 where its operator stores matrix values, FP64 where it does not (every route
-of this mix: the on-the-fly sigma, the block-staged and one-launch DOCI
+of this mix: the on-the-fly sigma, the block-staged and small-batch DOCI
 products), and it stops at a Kato-Temple energy estimate of 1e-9 Eh.  The timed stream holds
 --requests (4,096) requests; one step = one slice of requests/steps
 consecutive requests, and the K slices are served back to back.
@@ -79,7 +79,7 @@ def parse():
     p.add_argument("--no-fp64", action="store_true", help="direct16: skip the FP64 solve")
     p.add_argument("--cpu-lines", type=int, default=6, help="alpha lines in the FCI CPU-baseline sample")
     p.add_argument("--solver", choices=["auto", "lanczos", "davidson"], default="auto",
-                   help="stream: served solver (auto: DOCI up to 13,312 determinants in batched one-launch "
+                   help="stream: served solver (auto: DOCI up to 13,312 determinants in batched lock-step "
                         "solves, Davidson for FCI and larger DOCI)")
     return p.parse_args()
 
@@ -441,8 +441,8 @@ def bench_stream(a, CA):
         "config": {"workload": ("served stream of rotated-integral ground-state solves: 70% DOCI L~U[12,20], "
                                 "30% FCI L~U[8,11] (on-the-fly sigma), half filling, seeds 1000+k, U=exp(K) "
                                 f"K~N(0,0.05^2), {prec_note}, Kato-Temple energy stop 1e-9 Eh"),
-                   "solver": {"auto": ("DOCI <= 13,312 determinants: batched FP64 Lanczos, one workgroup per "
-                                       "request (cf_solve_doci_batch); FCI and larger DOCI: Davidson"),
+                   "solver": {"auto": ("DOCI <= 13,312 determinants: batched FP64 Lanczos in lock step "
+                                       "(cf_solve_doci_batch); FCI and larger DOCI: Davidson"),
                               "lanczos": "thick-restart Lanczos", "davidson": "Davidson"}[a.solver],
                    "requests": NREQ, "step": f"one slice of {NREQ}/{K} = {slice_sz:.1f} consecutive requests",
                    "warmup_requests": nwarm,

@@ -944,7 +944,7 @@ class SolveServer(_Handle):
 
 
 def solve_doci_batch(requests, ctx: "Context | None" = None) -> list[dict]:
-    """cf_solve_doci_batch: many small DOCI solves in one launch.  requests:
+    """cf_solve_doci_batch: many small DOCI solves in lock step.  requests:
     dicts with h, V, npair and optionally U, econst, tol, tol_energy,
     check_every, tag; returns one result dict per request (SolveServer.poll's
     fields)."""

@@ -1292,14 +1292,14 @@ int cf_crs_build(cf_space* sp, int value_prec, double zero, cf_crs** out) {
     }
     // DOCI matrices: the pair elements come from an L x L table in LDS instead
     // of the 8/12-byte element stream of the row gather.  Measured on MI355X
-    // (FP64 / FP32 values): L = 24 block-staged 0.262 / 0.262 ms, hop columns
-    // 0.472 / 0.477, row gather 1.468 / 1.076; L = 22 68 / 69 against 121 / 125
-    // (hop columns) and 312 / 226 us; L = 20 18.7 / 19.1 against 33.1 / 33.8
-    // and 73 / 52 us; L = 19 (92,378 rows) 15.8 / 15.7 against 21.1 / 21.5 and
-    // 31.7 / 23.7 us; L = 18 (48,620 rows) hop columns 13.2 against 14.5
-    // (block-staged) and 15.7 / 11.5 us (row gather).  Below that the launch
-    // dominates and the row gather is as fast, so smaller matrices build on
-    // request.
+    // (FP64 / FP32 values): L = 24 block-staged 0.174 / 0.167 ms, hop columns
+    // 0.471 / 0.476, row gather 1.47 / 1.07; L = 22 42 / 41 against 118 / 121
+    // (hop columns) and 304 / 220 us; L = 20 13.3 / 13.0 against 31 / 32 and
+    // 72 / 52 us; L = 19 (92,378 rows) 10.0 / 9.8 against 20.3 / 21.0 and
+    // 31 / 23 us; L = 18 (48,620 rows) 9.3 / 8.9 against 12.7 / 12.8 and
+    // 15.5 / 11.0 us; L = 17 (24,310) 8.9 / 8.7 against 8.0 / 7.9 and 7.1 / 6.3.
+    // Below that the launch dominates, so smaller matrices build on request.
+    // (The block-staged line stays at the 60,000 rows that ciflow_amd.h states.)
     if (sp->kind == CF_DOCI && m->n >= 40000) {
         const int L = sp->ham->L, w = doci_block_w(L);
         if (m->n >= 60000 && L - w <= 20) {

@@ -6,7 +6,7 @@
 // (OrbitalOptimization::update_cim -> set_ham -> build_ci -> solve,
 // SimulatedAnnealing.cpp:83-87).
 //
-// Lane l is grid row blockIdx.y (blockIdx.z for the dot products); its grid-x
+// Lane l is grid row blockIdx.y (blockIdx.z for the new column's dots); its grid-x
 // decomposition, and so every reduction order, depends on n alone, so a
 // lane's results are the same in any batch and alone.  The arithmetic of
 // each step is that of the single-request Davidson step kernels (krylov.hip):

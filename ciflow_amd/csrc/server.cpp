@@ -57,11 +57,11 @@ struct cf_server {
 };
 
 namespace {
-// Requests the batched one-launch DOCI solver takes (cf_solve_doci_batch):
+// Requests the batched small-DOCI solver takes (cf_solve_doci_batch):
 // the server's own choice (CF_SOLVER_AUTO), DOCI, a space of at most
 // kBatchN determinants.
 constexpr uint64_t kBatchN = 13312;
-constexpr size_t kBatchMax = 256;  // requests per batch (one workgroup each)
+constexpr size_t kBatchMax = 256;  // requests per batch
 
 bool batchable(const cf_request& r) {
     return r.kind == CF_DOCI && r.method == CF_SOLVER_AUTO && r.nup == r.ndown && r.nup >= 1 && r.nup < r.L &&
@@ -70,7 +70,7 @@ bool batchable(const cf_request& r) {
 
 // Requests the batched Davidson solver takes (cf_solve_batch): the server's
 // own choice (CF_SOLVER_AUTO), FCI on the on-the-fly sigma or DOCI above the
-// one-launch size, of a shape it has kernels for.
+// size of the small-DOCI solver, of a shape it has kernels for.
 constexpr size_t kDavBatchMax = 32;  // requests per lock-step batch
 
 bool dav_batchable(const cf_request& r) {
@@ -410,7 +410,7 @@ void worker_main(cf_server* S) {
 extern "C" {
 
 // CF_PREC_AUTO: FP32 values only where the request's route stores matrix
-// values (a stored CRS); the one-launch DOCI batch, the lock-step Davidson
+// values (a stored CRS); the small-DOCI batch, the lock-step Davidson
 // batch and the on-the-fly sigma read none, and FP64 is as fast or faster
 // there (measured per class on MI355X: FP64 lock-step batches 0-21% more
 // solves/s, the FP32 phase ending in 3-12 extra FP64 polish products).

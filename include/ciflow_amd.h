@@ -40,7 +40,7 @@ enum {
     CF_PREC_AUTO = 2 /* served requests (cf_server_submit, cf_solve_batch, cf_request_footprint)
                         only: CF_F32 where the request's operator reads stored matrix values (a
                         stored CRS: the FP32 copy halves the product's bytes), CF_F64 where it
-                        does not (the on-the-fly sigma, the block-staged and one-launch DOCI
+                        does not (the on-the-fly sigma, the block-staged and small-batch DOCI
                         products: measured equal or faster in FP64, the FP32 phase adding the
                         products of the FP64 polish) */
 };
@@ -393,7 +393,7 @@ typedef struct {
     int direct;         /* FCI only: 1 = on-the-fly sigma (cf_solve_direct) instead of a stored CRS */
     int method;         /* cf_solve_opts.method: CF_LANCZOS, CF_DAVIDSON, or CF_SOLVER_AUTO:
                            the server packs DOCI requests of at most 13,312
-                           determinants into batched one-launch solves
+                           determinants into batched solves
                            (cf_solve_doci_batch) and takes Davidson for FCI and
                            the larger DOCI ones */
 } cf_request;
@@ -407,12 +407,12 @@ typedef struct {
     double t_submit, t_start, t_end;  /* steady-clock seconds */
     char error[160];
 } cf_result;
-/* Many small DOCI solves in one launch (the loop above issues them one after
+/* Many small DOCI solves in lock step (the loop above issues them one after
  * another: OrbitalOptimization::update_cim -> set_ham -> build_ci -> solve,
  * SimulatedAnnealing.cpp:83-87): every request whose DOCI space has at most
- * 13,312 determinants (nalpha == nbeta, L <= 32) is solved by one workgroup
- * running FP64 Lanczos on the matrix of DOCI::construct_CI_matrix
- * (CIMethod.cpp:611-660) applied without storing it; the integrals are
+ * 13,312 determinants (nalpha == nbeta, L <= 32) is solved by FP64 Lanczos on
+ * the matrix of DOCI::construct_CI_matrix (CIMethod.cpp:611-660) applied
+ * without storing it, one launch a step for all of them; the integrals are
  * rotated by U (or taken as they are when U is NULL) in batched FP64-MFMA
  * transforms.  Stops as cf_solve_opts with tol (<= 0: 1e-12), tol_energy and
  * check_every (<= 0: 2); at most 400 products (solve_status 1 beyond).  The
