@@ -7,6 +7,7 @@ namespace cf {
 
 constexpr int kBatchMaxL = 32;        // orbitals
 constexpr int kBatchMaxSteps = 400;   // Lanczos steps (products) per request
+constexpr int kBatchRunning = 1 << 30;  // no step has given a result yet
 
 // One request of a batch (device memory).
 struct DociBatchJob {
@@ -19,7 +20,7 @@ struct DociBatchJob {
     uint64_t seed = 0;             // start vector
     double* out = nullptr;         // eigval, residual, products, status (0 converged, 1 step limit)
     double* scratch = nullptr;     // doci_batch_scratch(n, L) doubles
-    int* done = nullptr;           // set once the request has its result
+    int* done = nullptr;           // step whose launch gave the request its result (before: kBatchRunning)
     int L = 0, np = 0, nv = 0, n = 0;
     int check = 2;                 // convergence test every `check` steps (>= 1)
     int max_steps = kBatchMaxSteps;

@@ -189,9 +189,10 @@ struct Work {
     }
 };
 
-// Convergence test of T_m by the whole workgroup (two waves work); sets the
-// request's result and done flag when it stops.
-__device__ void lanczos_test(const DociBatchJob& J, int m, int maxs, TestMatrix& T, int count, int* left, int* flag) {
+// Convergence test of T_m, m = j - 1, by the whole workgroup (two waves work);
+// sets the request's result and the step it was found in when it stops.
+__device__ void lanczos_test(const DociBatchJob& J, int j, int maxs, TestMatrix& T, int count, int* left, int* flag) {
+    const int m = j - 1;
     const Work W(J);
     __shared__ double ctl[6];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -263,7 +264,7 @@ __device__ void lanczos_test(const DociBatchJob& J, int m, int maxs, TestMatrix&
             J.out[1] = r0;
             J.out[2] = (double)m;
             J.out[3] = stop ? 0.0 : 1.0;
-            *J.done = 1;
+            __hip_atomic_store(J.done, j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (atomicAdd(left, 1) + 1 == count) {
                 *flag = 1;  // host memory
                 __threadfence_system();
@@ -320,7 +321,7 @@ __global__ void __launch_bounds__(256) k_doci_batch_init(const DociBatchJob* __r
     for (int t = threadIdx.x; t < L; t += 256)
         d1[t] = 2.0 * J.h[t * L + t] + J.V[(((size_t)t * L + t) * L + t) * L + t];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *J.done = 0;
+        *J.done = kBatchRunning;
         W.al[kMaxSteps] = W.al[kMaxSteps + 1] = 1e300;  // no test yet
         if (blockIdx.y == 0) *left = 0;
     }
@@ -346,10 +347,12 @@ __global__ void __launch_bounds__(NT) k_doci_batch_step(const DociBatchJob* __re
     extern __shared__ __align__(16) unsigned char smem_batch[];
     __shared__ double red[NT / 64];
     const DociBatchJob& J = jobs[blockIdx.y];
-    if (*J.done) return;
+    // Finished in an earlier launch.  This launch's test may store j meanwhile, which
+    // counts as not finished: the whole workgroup decides alike, and barriers follow.
+    if (__hip_atomic_load(J.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < j) return;
     const int maxs = J.max_steps < kMaxSteps ? J.max_steps : kMaxSteps;
     if ((int)blockIdx.x == nchunk) {
-        if (j >= 2 && j - 1 <= maxs) lanczos_test(J, j - 1, maxs, *(TestMatrix*)smem_batch, count, left, flag);
+        if (j >= 2 && j - 1 <= maxs) lanczos_test(J, j, maxs, *(TestMatrix*)smem_batch, count, left, flag);
         return;
     }
     const int n = J.n, L = J.L, tid = threadIdx.x;

@@ -45,3 +45,17 @@ def test_more_requests_than_workgroups_fill_the_gpu():
     res = CA.solve_doci_batch([qs[k % 4] for k in range(1100)])   # one workgroup per request
     for k, r in enumerate(res):
         assert r["energy"] == alone[k % 4]["energy"] and r["n_matvec"] == alone[k % 4]["n_matvec"]
+
+
+def test_requests_that_finish_at_different_steps():
+    """An energy stop, the default tolerance and one that no residual meets, in one
+    launch sequence: early ones stay as they are alone while the last takes 400 steps."""
+    qs = [dict(request(12, 6, 700), tol_energy=1e-3), request(12, 6, 701), dict(request(12, 5, 702), tol=1e-300),
+          dict(request(8, 4, 703), tol_energy=1e-9), dict(request(12, 6, 704), tol=1e-6)]
+    alone = [CA.solve_doci_batch([q])[0] for q in qs]
+    assert [r["solve_status"] for r in alone] == [0, 0, 1, 0, 0] and alone[2]["n_matvec"] == 400
+    assert len({r["n_matvec"] for r in alone}) >= 4
+    for _ in range(3):
+        for a, r in zip(alone, CA.solve_doci_batch(qs)):
+            assert all(a[k] == r[k] for k in ("energy", "resid", "n_matvec", "solve_status"))
+    assert abs(alone[2]["energy"] - stored_energy(qs[2])) <= 1e-10
