@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "built_map.h"
 #include "capi_types.h"
 #include "dets.h"
 #include "kernels.h"
@@ -2473,24 +2474,24 @@ int cf_solve_doci_batch(cf_ctx* ctx, int count, const cf_request* reqs, cf_resul
         }
     }
     // shared tables of each (L, pairs) shape, built once per context
+    std::vector<const cf_ctx::DociTables*> tabs(count, nullptr);
     for (int i = 0; i < count; ++i) {
         if (!ok[i]) continue;
         const int L = reqs[i].L, np = reqs[i].nup;
-        auto key = std::make_pair(L, np);
-        if (ctx->doci_tabs.count(key)) continue;
-        cf_ctx::DociTables& T = ctx->doci_tabs[key];
-        const uint64_t n = binom_host(L, np);
-        T.s.alloc(n);
-        T.col.alloc(n * (uint64_t)np * (L - np));
-        launch_unrank(L, np, 0, n, ctx->binom.p, T.s.p, st);
-        DociEllArgs a;
-        a.n = n;
-        a.L = L;
-        a.np = np;
-        a.nv = L - np;
-        a.s = T.s.p;
-        launch_doci_ell_fill(a, ctx->binom.p, T.col.p, st);
-        launch_doci_hops(T.s.p, n, L, np, T.col.p, st);
+        tabs[i] = &built_entry(ctx->doci_tabs, std::make_pair(L, np), [&](cf_ctx::DociTables& T) {
+            const uint64_t n = binom_host(L, np);
+            T.s.alloc(n);
+            T.col.alloc(n * (uint64_t)np * (L - np));
+            launch_unrank(L, np, 0, n, ctx->binom.p, T.s.p, st);
+            DociEllArgs a;
+            a.n = n;
+            a.L = L;
+            a.np = np;
+            a.nv = L - np;
+            a.s = T.s.p;
+            launch_doci_ell_fill(a, ctx->binom.p, T.col.p, st);
+            launch_doci_hops(T.s.p, n, L, np, T.col.p, st);
+        });
     }
     // jobs by size class: one lock-step batch each
     uint64_t scratch_n = 0;
@@ -2514,9 +2515,8 @@ int cf_solve_doci_batch(cf_ctx* ctx, int count, const cf_request* reqs, cf_resul
             DociBatchJob J;
             J.h = hptr[i];
             J.V = vptr[i];
-            const cf_ctx::DociTables& T = ctx->doci_tabs[std::make_pair(r.L, r.nup)];
-            J.s = T.s.p;
-            J.hops = T.col.p;
+            J.s = tabs[i]->s.p;
+            J.hops = tabs[i]->col.p;
             J.tol = r.tol > 0 ? r.tol : dflt.tol;
             J.tol_energy = r.tol_energy > 0 ? r.tol_energy : 0.0;
             J.seed = dflt.seed;

@@ -16,6 +16,7 @@
 // phase and stops; a finished lane idles), the host keeps each lane's
 // projected matrix, and a lane's device arithmetic depends on n alone, so a
 // request's result is the same in any batch and alone.
+#include "built_map.h"
 #include "davbatch.h"
 
 #include <algorithm>
@@ -129,9 +130,9 @@ void Batch::alloc() {
     hop.assign(cap, BdOpLane{});
     hargs.assign(cap, SigmaArgs{});
     if (kind == CF_DOCI) {
-        auto key = std::make_pair(L, nup);
-        if (!c->doci_blk.count(key)) make_doci_block_tables(c, L, nup, doci_block_w(L), c->doci_blk[key]);
-        blk = &c->doci_blk[key];
+        blk = &built_entry(c->doci_blk, std::make_pair(L, nup), [&](cf_ctx::DociBlockTables& T) {
+            make_doci_block_tables(c, L, nup, doci_block_w(L), T);
+        });
         blk->args.zero = kDociZero;
     }
     const size_t Bn = (size_t)cap * n;
