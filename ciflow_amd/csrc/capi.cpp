@@ -334,10 +334,10 @@ bool make_sell(cf_crs* m, bool optional = false) {
         free_b += block_budget(c->device)->held();  // kept blocks are given back when memory runs out
         if (entries * (12 + (m->want32 ? 4 : 0)) > free_b / 2) return false;
     }
-    if (m->scol.n != entries) {
-        m->scol.alloc(entries);
+    if (m->scol.n != entries) {  // scol last: its size says that all of them are there
         m->sval.alloc(entries);
         if (m->want32) m->sval32.alloc(entries);
+        m->scol.alloc(entries);
     }
     if (!m->spart.p && m->n < (1ull << 21)) m->spart.alloc(kSellMaxSplit * m->n);
     KTimer t(c, "crs_fill");
@@ -406,9 +406,10 @@ void make_doci_table(cf_crs* m) {
     a.s = sp->ta->s.p;
     a.diag = sp->diag.p;
     a.zero = m->zero;
-    m->dvk.alloc((uint64_t)a.L * a.L);
+    DBuf<double> vk((uint64_t)a.L * a.L);
     m->dvk32.alloc((uint64_t)a.L * a.L);
-    launch_doci_pair_table(a, H->dev(), m->dvk.p, m->dvk32.p, H->ctx->stream);
+    launch_doci_pair_table(a, H->dev(), vk.p, m->dvk32.p, H->ctx->stream);
+    m->dvk = std::move(vk);  // last: it says that the tables are there
 }
 
 void make_doci_ell(cf_crs* m) {
