@@ -113,8 +113,12 @@ __global__ void __launch_bounds__(256) k_mfma_gather(uint64_t db, int Sb, int ro
     for (; n < end; ++n) gat[(uint64_t)n * db + Ib] = (uint32_t)(rows * kFS) * 8u;  // the row of zeros
 }
 
-// *sym = 1 if V[p][q][r][s] = V[p][s][r][q] to 2e-14 of the largest element
-// (integrals over real orbitals; rotated ones differ by rounding).
+// *sym = 1 if V[p][q][r][s] = V[p][s][r][q] to rounding: 2^-50 of the largest
+// element.  Integrals over real orbitals, whose rotations differ by 5.1e-16 of it
+// at most (L = 4 .. 16, six sets, small and large rotations).  The product takes
+// the mean of the two, so what it takes differs from what it was given by half
+// of that: 1e-16 relative in the result of rotated integrals, below its sums'
+// rounding.
 __global__ void __launch_bounds__(1024) k_v_symmetric(int L, const double* __restrict__ V, int* sym) {
     __shared__ double red[16];
     __shared__ int bad;
@@ -127,7 +131,7 @@ __global__ void __launch_bounds__(1024) k_v_symmetric(int L, const double* __res
     if (threadIdx.x == 0) bad = 0;
     __syncthreads();
     for (int i = 0; i < 16; ++i) m = fmax(m, red[i]);
-    const double most = 2e-14 * m;
+    const double most = 0x1p-50 * m;
     for (int i = threadIdx.x; i < L4; i += 1024) {
         const int p = i / (L2 * L), q = i / L2 % L, r = i / L % L, s = i % L;
         if (q > s && !(fabs(V[i] - V[((p * L + s) * L + r) * L + q]) <= most)) bad = 1;
@@ -178,7 +182,7 @@ __global__ void __launch_bounds__(kThreads, RT <= 4 && KS <= 8 ? 4 : 2)
             for (int k = 0; k < KS; ++k) av[t][k] = j < db ? row[k][j] : 0.0;
         }
     }
-    // B[a][{qs}] = s_a V[p_a][q][r_a][s], zeros past the actions and pairs
+    // B[a][{qs}] = s_a V[p_a][q][r_a][s] (the mean of the two orders), zeros past the actions and pairs
     for (int e = w; e < KS * 4; e += kWaves) {
         const Exc x = la[e < Sa ? e : 0];
         const double* v = x.type == 0 ? a.vself64 + (uint64_t)Ia * L2 : a.vpair64 + (uint64_t)(x.f * L + x.t) * L2;
@@ -187,7 +191,8 @@ __global__ void __launch_bounds__(kThreads, RT <= 4 && KS <= 8 ? 4 : 2)
             double y = 0.0;
             if (e < Sa && c < m.np) {
                 const int q = (int)((sqrtf(8 * c + 1.5f) - 1.0f) * 0.5f);  // c >= q (q + 1) / 2
-                y = v[q * L + c - q * (q + 1) / 2];
+                const int s = c - q * (q + 1) / 2;
+                y = 0.5 * (v[q * L + s] + v[s * L + q]);
             }
             B[e * m.bs + c] = neg ? -y : y;
         }

@@ -316,7 +316,7 @@ int cf_sigma_set_threads(cf_sigma* s, int threads);
  * action's V slice and C row, 2 = per-Hamiltonian slice tables with the next
  * action's slice and row prefetched into registers (shapes it does not cover
  * run kernel 1), 3 (default) = in FP64, for V[p][q][r][s] = V[p][s][r][q] (real
- * orbitals) and up to 1,024 beta strings, a matrix product over the alpha
+ * orbitals; to 2^-50 of the largest element) and up to 1,024 beta strings, a matrix product over the alpha
  * actions; otherwise kernel 2 with packed LDS offsets and exact beta-list
  * lengths (shapes without an instance run kernel 2). */
 int cf_sigma_set_kernel(cf_sigma* s, int kernel);

@@ -52,3 +52,19 @@ def test_integrals_without_the_symmetry():
         ci = CA.FCI(CA.Hamiltonian(q["h"], q["V"], 4, 4))
         ci.solve()
         assert abs(ci.get_ci_energy() - r["energy"]) <= 1e-10
+
+
+@pytest.mark.parametrize("size", [9e-15, 2e-15, 2e-16])
+def test_integrals_that_are_nearly_symmetric(size):
+    """A Hermitian part that is antisymmetric in q <-> s (the two orders differ by twice its
+    size) is used as given unless it is rounding."""
+    L = 8
+    h, V = CA.gen_integrals(L, 77)
+    K = np.triu(np.ones((L, L)), 1)
+    K -= K.T
+    V = V + size * np.abs(V).max() * np.einsum("pr,qs->pqrs", K, K)
+    ham = CA.Hamiltonian(h, V, 4, 4)
+    x = np.random.default_rng(8).standard_normal(4900)
+    z = CA.FCI(ham).get_mat().mvprod(x)
+    y = CA.FCI_Direct(ham).mvprod(x)
+    assert np.linalg.norm(y - z) <= 4e-15 * np.linalg.norm(z)
