@@ -98,13 +98,15 @@ __device__ __forceinline__ int sturm_count(const TestMatrix& T, int m, double x)
 // `prev`: that eigenvalue of an earlier T (any value above 1: none).  It is an
 // upper bound (interlacing), and the first round's points lie at distances
 // below it that grow 1.75-fold from lane to lane, so near convergence four
-// rounds are saved.  The tests take the value to 1e-13, which the last
-// component and the gap need; a result is refined to 1e-16.
-__device__ double kth_eigenvalue(const TestMatrix& T, int m, int k, double prev, double width) {
+// rounds are saved.  The value is taken to rounding (two units of the last
+// place): the last component moves by a hundred times its error, 5e-12 of the
+// residual estimate when it was taken to 1e-13, 3e-14 now, as much as the
+// rounding of T moves it.
+__device__ double kth_eigenvalue(const TestMatrix& T, int m, int k, double prev) {
     const int lane = threadIdx.x & 63;
     double lo = -1.0, hi = 1.0;
     const bool warm = prev < 1.0;
-    for (int round = 0; round < 13 && hi - lo > width; ++round) {
+    for (int round = 0; round < 13 && hi - lo > 2.5e-16; ++round) {
         const bool w = warm && round == 0;
         const double x = w ? prev - exp2(1.0 - 51.0 * (double)lane / 63.0) : lo + (hi - lo) * (double)(lane + 1) / 65.0;
         // the first lane whose point has more than k eigenvalues below it
@@ -225,7 +227,7 @@ __device__ void lanczos_test(const DociBatchJob& J, int j, int maxs, TestMatrix&
     __syncthreads();
     double* last_th = W.al + kMaxSteps;  // theta_0 and theta_1 of the last test
     if (wv < 2 && wv < m) {  // theta_0 and theta_1 at the same time
-        const double xk = kth_eigenvalue(T, m, wv, (last_th[wv] - mid) * rh, 1e-13);
+        const double xk = kth_eigenvalue(T, m, wv, (last_th[wv] - mid) * rh);
         if (lane == 0) {
             ctl[wv] = xk;
             last_th[wv] = mid + half * xk;
@@ -243,7 +245,7 @@ __device__ void lanczos_test(const DociBatchJob& J, int j, int maxs, TestMatrix&
             break;
         }
         if (wv == 0) {
-            const double xk = kth_eigenvalue(T, m, k1, 2.0, 1e-13);
+            const double xk = kth_eigenvalue(T, m, k1, 2.0);
             if (lane == 0) ctl[1] = xk;
         }
         __syncthreads();
@@ -257,18 +259,15 @@ __device__ void lanczos_test(const DociBatchJob& J, int j, int maxs, TestMatrix&
         const double mu = th1 - r1;
         stop = mu > th0 && r0 * r0 <= J.tol_energy * (mu - th0);
     }
-    if ((stop || m == maxs) && wv == 0) {
-        const double xf = kth_eigenvalue(T, m, 0, x0, 1e-16);
-        if (lane == 0) {
-            J.out[0] = mid + half * xf;
-            J.out[1] = r0;
-            J.out[2] = (double)m;
-            J.out[3] = stop ? 0.0 : 1.0;
-            __hip_atomic_store(J.done, j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (atomicAdd(left, 1) + 1 == count) {
-                *flag = 1;  // host memory
-                __threadfence_system();
-            }
+    if ((stop || m == maxs) && tid == 0) {
+        J.out[0] = th0;
+        J.out[1] = r0;
+        J.out[2] = (double)m;
+        J.out[3] = stop ? 0.0 : 1.0;
+        __hip_atomic_store(J.done, j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (atomicAdd(left, 1) + 1 == count) {
+            *flag = 1;  // host memory
+            __threadfence_system();
         }
     }
 }
