@@ -312,9 +312,11 @@ void launch_finish_step_r(uint64_t n, int j, const double* c1, const double* c2,
 // each forms alpha_j = v_j . w and w' = w - alpha_j v_j - beta_{j-1} v_{j-1} itself
 // (4 n doubles from L2) and then its own c_g = v_g . w', so nothing waits for a
 // partial sum.  k_step_next removes the c and normalises at once: the basis is
-// orthonormal, so |w' - V c|^2 = |w'|^2 - |c|^2, exact to rounding while the c
-// are the small corrections they are here; if they hold more than half of w' (next
-// to a breakdown) every workgroup sums the norm from the vector instead.
+// orthonormal, so |w' - V c|^2 = |w'|^2 - |c|^2, as good as a sum over the vector
+// while the c are the corrections that they are here (1e-30 of w'^2 together); if
+// they hold more than 2^-20 of it (next to a breakdown), so that the difference would
+// lose something (7.4e-16 of beta at a share of a half, 1.5e-16 for the vector's
+// own sum), every workgroup sums the norm from the vector instead.
 // FCI L=8 (4,900 rows): 36 us a step with its product, 27 of them in five
 // launches, now 19 (6.1 + 4.3 us and 8.9 for the product); DOCI L=10 (252) 23 ->
 // 10 us.  An optimisation step of the two: 4.8 -> 2.85 and 2.07 -> 1.19 ms.  From
@@ -401,7 +403,7 @@ __global__ void __launch_bounds__(256) k_step_next(int n, int j, const double* _
     const int q = blockIdx.x * 256 + tid;
     const double x = q < n ? corrected(q) : 0.0;
     double b2 = w2 - c2;
-    if (!(c2 <= 0.5 * w2)) {  // uniform over the grid
+    if (!(c2 <= 0x1p-20 * w2)) {  // uniform over the grid
         double m = 0.0;
         for (int t = tid; t < n; t += 256) {
             const double y = corrected(t);
