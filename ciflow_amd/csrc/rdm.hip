@@ -654,9 +654,14 @@ void rdm_dense(hipStream_t stream, int kind, int L, int nup, int ndown, uint64_t
     std::vector<double> g(2 * (size_t)P, 0.0);
     if (kind == 1) {  // DOCI
         // 16 rows a workgroup while that fills the GPU: each thread's bin is a
-        // serial loop over them (252 rows in one workgroup took 151 us)
+        // serial loop over them (252 rows in one workgroup took 151 us).  With the
+        // pair bins, whose terms wait for a gather, long loops want twice as many
+        // (512 / 1,024 workgroups: L=18 0.37 / 0.36 ms, L=20 0.67 / 0.56, L=22 2.64 /
+        // 2.16, L=24 13.4 / 12.1); without them the shorter sum over chunks wins
+        // (L=18 0.085 / 0.107 ms, L=20 0.167 / 0.180, L=24 1.47 / 1.45)
         uint64_t nchunk = (n + 15) / 16;
-        if (nchunk > 512) nchunk = 512;
+        const uint64_t most = Gamma && n >= 100000 ? 1024 : 512;
+        if (nchunk > most) nchunk = most;
         if (nchunk < 1) nchunk = 1;
         const uint64_t rows = (n + nchunk - 1) / nchunk;
         const uint64_t len = 2 * (uint64_t)P + L;
