@@ -312,7 +312,7 @@ static void rdm_from_x(hipStream_t stream, int L, uint64_t n, const double* c, c
 }
 
 // ---------------------------------------------------------------------------
-// FCI densities from one-spin matrices (L <= 16, string spaces of <= 16,384).
+// FCI densities from one-spin matrices (L <= 16).
 //
 // For a fixed alpha string ka the transition densities X^a(ka, kb)_rp = s
 // c(J, kb) are rows of C with the string J = ka - r + p and the same for every
@@ -702,8 +702,14 @@ void rdm_dense(hipStream_t stream, int kind, int L, int nup, int ndown, uint64_t
         }
         return;
     }
-    // FCI: one-spin matrices where they are small (2 GiB at most), else X in memory
-    if (L <= 16 && da <= 16384 && db <= 16384) {
+    // FCI up to L = 16 (12,870 strings a spin): one-spin matrices; at most 1.3 GB for
+    // one of them and, with the 2-RDM, 1.9 GB of opposite-spin blocks beside the
+    // vector.  Above, X in memory, and for the 1-RDM alone of a space with hardly
+    // any strings of one spin: X has n L^2 entries then where the matrix has d^2 (one-spin
+    // / X, ms: L=16 8a0b d^2 = 50 n L^2 1.29 / 0.61, 6a0b 31 n L^2 0.72 / 0.59, L=15 7a0b 29
+    // 0.53 / 0.56, L=14 7a0b 17 0.29 / 0.49, L=16 8a1b 3 1.37 / 1.48)
+    const bool narrow = !Gamma && da * da + db * db > 30 * n * (uint64_t)P;
+    if (L <= 16 && !narrow) {
         rdm_fci(stream, L, nup, ndown, da, db, sa, sb, suba, subb, Sa, Sb, c.p, gamma, Gamma);
         return;
     }

@@ -1,7 +1,9 @@
 """GPU tests of the FCI densities from one-spin matrices: every size at an edge
 of its tiles (64 strings, 32 beta strings a stage, 16 columns) against <a+a> and
 <a+a+aa> contracted from plain numpy transition densities, with unequal spins,
-empty and full shells, the 1-RDM alone, and an unnormalised vector."""
+empty and full shells, the 1-RDM alone, and an unnormalised vector; and of the
+ones that go through transition densities in memory (L > 16; the 1-RDM of a space
+with many strings of one spin and hardly any of the other)."""
 from math import comb
 
 import numpy as np
@@ -52,7 +54,8 @@ def reference(L, na, nb, c):
 
 
 @pytest.mark.parametrize("L,na,nb", [(1, 1, 0), (3, 0, 2), (3, 3, 1), (4, 2, 2), (6, 3, 1), (7, 2, 5), (8, 4, 3),
-                                     (9, 2, 4), (10, 1, 5), (11, 3, 2), (12, 2, 3), (13, 2, 2), (16, 1, 2)])
+                                     (9, 2, 4), (10, 1, 5), (11, 3, 2), (12, 2, 3), (13, 2, 2), (16, 1, 2),
+                                     (17, 1, 2), (18, 2, 1), (16, 6, 0)])
 def test_densities(L, na, nb):
     h, V = CA.gen_integrals(max(L, 2), 3)
     h, V = h[:L, :L].copy(), V[:L, :L, :L, :L].copy()
