@@ -136,6 +136,7 @@ def lib():
         "cf_ctx_create": (C.c_int, [C.c_int, C.POINTER(vp)]),
         "cf_ctx_destroy": (C.c_int, [vp]),
         "cf_ctx_synchronize": (C.c_int, [vp]),
+        "cf_ctx_trim": (C.c_int, [vp, u64p]),
         "cf_ctx_enable_timing": (C.c_int, [vp, C.c_int]),
         "cf_ctx_kernel_time": (C.c_int, [vp, C.c_char_p, C.POINTER(C.c_int64), dp]),
         "cf_ctx_reset_timing": (C.c_int, [vp]),
@@ -270,6 +271,13 @@ class Context:
 
     def synchronize(self):
         _check(lib().cf_ctx_synchronize(self.ptr))
+
+    def trim(self) -> int:
+        """Gives the device memory kept for reuse on this context's device back to
+        the device (for torch or another process); returns its bytes."""
+        b = C.c_uint64()
+        _check(lib().cf_ctx_trim(self.ptr, C.byref(b)))
+        return b.value
 
     def enable_timing(self, on: bool = True):
         _check(lib().cf_ctx_enable_timing(self.ptr, int(on)))

@@ -17,7 +17,9 @@
 // bounded over all caches of a device; a block past the bound pushes out the
 // cache's oldest ones or goes back itself, one that was not reused for
 // kKeepTakes requests goes back, an allocation that fails first takes back
-// what every cache of the device holds, and close() returns the rest.
+// what every cache of the device holds, and close() returns the rest.  What other
+// libraries and processes on the device need is not seen here: a large block is
+// not kept while the device is short of memory, and cf_ctx_trim gives back all.
 //
 // No HIP in this file: the policy is tested on the CPU with a source of its own.
 #pragma once
@@ -41,6 +43,7 @@ struct BlockSource {
     virtual void free(void* p) = 0;               // after the work enqueued so far
     virtual void free_unordered(void* p) = 0;     // once the owner (its stream) is gone
     virtual void drain() = 0;                     // until freed blocks are really back
+    virtual bool scarce() { return false; }       // others of the device may need a block more than we do
 };
 
 class BlockCache;
@@ -65,12 +68,13 @@ struct BlockBudget {
         std::lock_guard<std::mutex> lk(cached_mu);
         return cached;
     }
-    inline void trim_all();
+    inline uint64_t trim_all();  // bytes given back
 };
 
 class BlockCache {
   public:
     static constexpr uint64_t kKeepTakes = 4096;
+    static constexpr size_t kLarge = 32u << 20;  // blocks worth a look at the device's free memory
 
     BlockCache(BlockSource* src, BlockBudget* budget) : src_(src), budget_(budget) {
         std::lock_guard<std::mutex> lk(budget_->mu);
@@ -110,6 +114,10 @@ class BlockCache {
             return;
         }
         while (!age_.empty() && takes_ - age_.front().take > kKeepTakes) src_->free(evict());
+        if (bytes >= kLarge && src_->scarce()) {
+            src_->free(p);
+            return;
+        }
         bool kept = budget_->reserve(bytes);
         while (!kept && bytes <= budget_->limit && !age_.empty()) {
             src_->free(evict());
@@ -130,10 +138,15 @@ class BlockCache {
         src_->free(p);
     }
 
-    // Every kept block goes back.
-    void trim() {
+    // Every kept block goes back; their bytes.
+    uint64_t trim() {
         std::lock_guard<std::mutex> lk(mu_);
-        while (!age_.empty()) src_->free(evict());
+        uint64_t bytes = 0;
+        while (!age_.empty()) {
+            bytes += age_.front().bytes;
+            src_->free(evict());
+        }
+        return bytes;
     }
 
     // Every kept block goes back, and blocks given later go straight back.
@@ -189,12 +202,14 @@ class BlockCache {
     bool closed_ = false;
 };
 
-inline void BlockBudget::trim_all() {
+inline uint64_t BlockBudget::trim_all() {
     std::lock_guard<std::mutex> lk(mu);
+    uint64_t bytes = 0;
     for (BlockCache* c : caches) {
-        c->trim();
+        bytes += c->trim();
         c->drain();
     }
+    return bytes;
 }
 
 }  // namespace cf

@@ -1024,6 +1024,15 @@ int cf_ctx_synchronize(cf_ctx* ctx) {
     API_END
 }
 
+int cf_ctx_trim(cf_ctx* ctx, uint64_t* bytes) {
+    API_BEGIN
+    CF_REQUIRE(ctx, "ctx is NULL");
+    ctx->use();
+    const uint64_t b = block_budget(ctx->device)->trim_all();
+    if (bytes) *bytes = b;
+    API_END
+}
+
 int cf_ctx_enable_timing(cf_ctx* ctx, int enable) {
     API_BEGIN
     CF_REQUIRE(ctx, "ctx is NULL");

@@ -74,7 +74,12 @@ struct cf_ctx {
 
     rocblas_handle blas() {
         if (!blas_) {
-            if (rocblas_create_handle(&blas_) != rocblas_status_success) {
+            rocblas_status st = rocblas_create_handle(&blas_);
+            if (st != rocblas_status_success) {  // its workspace may need what the caches keep
+                cf::block_budget(device)->trim_all();
+                st = rocblas_create_handle(&blas_);
+            }
+            if (st != rocblas_status_success) {
                 blas_ = nullptr;
                 throw Error(ERR_HIP, "rocblas_create_handle failed");
             }
@@ -194,8 +199,6 @@ struct cf_sigma {
 };
 
 namespace cf {
-// The device's block caches and what they may keep together (1/16 of its memory).
-BlockBudget* block_budget(int device);
 // One-string diagonal parts and excitation lists of a string table for H.
 void fill_strtab(cf_ctx* ctx, const cf_ham* H, StrTab* t);
 // Diagonal of the space for its current Hamiltonian.

@@ -6,6 +6,7 @@
 #include "block_cache.h"
 #include "errors.h"
 
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <memory>
@@ -40,6 +41,23 @@ struct HipBlockSource : BlockSource {
     void free(void* p) override { (void)hipFreeAsync(p, stream); }
     void free_unordered(void* p) override { (void)hipFree(p); }
     void drain() override { (void)hipStreamSynchronize(stream); }
+    // less than an eighth of the device free (kept blocks count as used), asked for
+    // every 10 ms at most: 4 us a call, which a matrix build would make ten times
+    bool scarce() override {
+        const auto now = std::chrono::steady_clock::now();
+        if (now < next_look) return is_scarce;
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        next_look = now + std::chrono::milliseconds(10);
+        return is_scarce = free_b < total_b / 8;
+    }
+
+  private:  // read and written under the cache's lock
+    std::chrono::steady_clock::time_point next_look{};
+    bool is_scarce = false;
 };
 struct DeviceBlocks {
     HipBlockSource src;
@@ -51,6 +69,26 @@ struct DeviceBlocks {
 // context makes its own current here, so allocating and freeing neither
 // blocks the host nor waits for other streams.  Null: plain hipMalloc / hipFree.
 inline thread_local std::shared_ptr<DeviceBlocks> tls_blocks;
+
+// The device's block caches and what they may keep together (1/16 of its memory).
+BlockBudget* block_budget(int device);
+
+// hipMalloc for memory outside of the caches: one that fails takes back what they keep.
+inline void* device_malloc(size_t bytes) {
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        int device = 0;
+        CF_HIP(hipGetDevice(&device));
+        block_budget(device)->trim_all();
+        e = hipMalloc(&p, bytes);
+    }
+    if (e == hipSuccess) return p;
+    (void)hipGetLastError();
+    if (e == hipErrorOutOfMemory) throw Error(ERR_NOMEM, "device memory: " + std::to_string(bytes) + " bytes");
+    throw Error(ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
+}
 
 // Owning device buffer.
 template <class T>
@@ -86,7 +124,7 @@ struct DBuf {
                 if (!p) throw Error(ERR_NOMEM, "device memory: " + std::to_string(count * sizeof(T)) + " bytes");
                 s = tls_blocks;
             } else {
-                CF_HIP(hipMalloc((void**)&p, count * sizeof(T)));
+                p = (T*)device_malloc(count * sizeof(T));
             }
         }
         n = count;

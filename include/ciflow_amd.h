@@ -59,6 +59,11 @@ const char* cf_last_error(void);
 int cf_ctx_create(int device, cf_ctx** out);
 int cf_ctx_destroy(cf_ctx* ctx);
 int cf_ctx_synchronize(cf_ctx* ctx);
+/* Device memory that this library keeps for reuse on the context's device (all
+ * of its contexts there, at most 1/16 of the memory) goes back to the device,
+ * for other libraries and processes; *bytes (may be NULL) says how much.  Its own
+ * allocations do this by themselves when memory runs out.  Live buffers stay. */
+int cf_ctx_trim(cf_ctx* ctx, uint64_t* bytes);
 /* Per-kernel event timing on the context stream: enable, then read the
  * number of timed launches and their summed duration (ms) for a kernel
  * family: "spmv_f64", "spmv_f32", "crs_count", "crs_fill", "sigma", "rdm". */

@@ -45,7 +45,9 @@ struct HostSource : BlockSource {
         ++unordered;
         free(p);
     }
+    bool short_of = false;
     void drain() override { ++drains; }
+    bool scarce() override { return short_of; }
 };
 
 int main() {
@@ -78,8 +80,25 @@ int main() {
         q = c.take(big - (1u << 20), &g2);
         CHECK(q == p && g2 == big);
         c.give(q, g2);
-        c.trim();
-        CHECK(src.live.empty() && bud.held() == 0);
+        const size_t held = bud.held();
+        CHECK(held > 0 && c.trim() == held);
+        CHECK(src.live.empty() && bud.held() == 0 && c.trim() == 0);
+    }
+    {  // a device short of memory: large blocks are not kept, small ones are
+        BlockBudget bud;
+        bud.limit = 1 << 30;
+        HostSource src;
+        src.short_of = true;
+        BlockCache c(&src, &bud);
+        size_t g, h;
+        void *p = c.take(BlockCache::kLarge, &g), *q = c.take(BlockCache::kLarge - 256, &h);
+        c.give(p, g);
+        c.give(q, h);
+        CHECK(!src.live.count(p) && src.live.count(q) && bud.held() == h);
+        src.short_of = false;
+        p = c.take(BlockCache::kLarge, &g);
+        c.give(p, g);
+        CHECK(bud.held() == g + h && bud.trim_all() == g + h && src.live.empty());
     }
     {  // the bound: oldest blocks go first, a block over the bound goes at once
         BlockBudget bud;
