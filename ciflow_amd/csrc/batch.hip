@@ -475,11 +475,16 @@ void run_class(const DociBatchJob* d_jobs, int count, int max_n, int max_L, int 
 
 void run_doci_batch(const DociBatchJob* d_jobs, int count, int max_n, int max_L, int max_steps, int* left,
                     volatile int* flag, hipEvent_t ev[2], hipStream_t s) {
-    if (count <= 0) return;
-    if (max_n <= 1024) run_class<256, 4>(d_jobs, count, max_n, max_L, max_steps, left, flag, ev, s);
-    else if (max_n <= 4096) run_class<512, 8>(d_jobs, count, max_n, max_L, max_steps, left, flag, ev, s);
-    else if (max_n <= 1024 * 13) run_class<1024, 13>(d_jobs, count, max_n, max_L, max_steps, left, flag, ev, s);
-    else throw Error(ERR_UNSUPPORTED, "batched DOCI solve: more than 13,312 determinants");
+    if (max_n > 1024 * 13) throw Error(ERR_UNSUPPORTED, "batched DOCI solve: more than 13,312 determinants");
+    // requests are grid rows: the device states 65,536 of them, so larger batches run
+    // in parts (each request's sums are its own, so its result is the same)
+    constexpr int kMost = 32768;
+    for (int a = 0; a < count; a += kMost) {
+        const int k = std::min(kMost, count - a);
+        if (max_n <= 1024) run_class<256, 4>(d_jobs + a, k, max_n, max_L, max_steps, left, flag, ev, s);
+        else if (max_n <= 4096) run_class<512, 8>(d_jobs + a, k, max_n, max_L, max_steps, left, flag, ev, s);
+        else run_class<1024, 13>(d_jobs + a, k, max_n, max_L, max_steps, left, flag, ev, s);
+    }
 }
 
 }  // namespace cf

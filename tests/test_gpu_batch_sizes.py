@@ -93,3 +93,12 @@ def test_residual_estimates():
             r = CA.solve_doci_batch([q])[0]
             want = lanczos_residual(q, r["n_matvec"])
             assert abs(r["resid"] - want) <= 1e-13 * want, (L, seed, r["n_matvec"], r["resid"] / want - 1)
+
+
+def test_more_requests_than_a_grid_dimension():
+    q = request(2, 1, 600)
+    alone = CA.solve_doci_batch([q])[0]
+    res = CA.solve_doci_batch([q] * 70000)
+    assert len(res) == 70000
+    for r in res:
+        assert r["status"] == 0 and r["energy"] == alone["energy"] and r["n_matvec"] == alone["n_matvec"]
