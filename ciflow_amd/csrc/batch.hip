@@ -450,6 +450,12 @@ void run_class(const DociBatchJob* d_jobs, int count, int max_n, int max_L, int 
     const int nchunk = std::max(1, std::min((max_n + NT - 1) / NT, (1024 + count - 1) / count));
     int* dflag = nullptr;
     CF_HIP(hipHostGetDevicePointer((void**)&dflag, const_cast<int*>(flag), 0));
+    // what is queued writes `flag` and the requests' scratch: the caller reads the
+    // results and reuses both, also after a launch that throws, only when it has run
+    struct Drain {
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{s};
     *flag = 0;
     k_doci_batch_init<<<dim3((unsigned)((max_n + 255) / 256), (unsigned)count), 256, 0, s>>>(d_jobs, left);
     CF_HIP(hipGetLastError());
@@ -467,8 +473,6 @@ void run_class(const DociBatchJob* d_jobs, int count, int max_n, int max_L, int 
             if (*flag) break;
         }
     }
-    // what is still queued writes `flag` and the requests' scratch: the
-    // caller reads the results and reuses both only after it has run
     CF_HIP(hipStreamSynchronize(s));
 }
 }  // namespace
