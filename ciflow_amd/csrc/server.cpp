@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "../../include/ciflow_amd.h"
+#include "batch.h"
 #include "capi_types.h"
 #include "common.h"
 #include "davbatch.h"
@@ -100,7 +101,8 @@ uint64_t estimate_footprint(const cf_request& r) {
         const uint64_t dense = (da * da + (r.nup == r.ndown ? 0 : db * db)) * 8;
         return (uint64_t)(ncv + 3) * n * 8 + dense + n * 4 + (da + db) * 4096 + ints + (64ull << 20);
     }
-    if (batchable(r)) return 3 * da * 8 + 2 * ints + (1ull << 20);  // scratch + integrals (tables shared)
+    // scratch + integrals (tables shared)
+    if (batchable(r)) return cf::doci_batch_scratch(da, L) * 8 + 2 * ints + (1ull << 20);
     uint64_t n, row;
     if (r.kind == CF_DOCI) {
         n = da;
@@ -118,10 +120,20 @@ uint64_t estimate_footprint(const cf_request& r) {
     // FCI spaces without the position-major copy keep a sliced copy of the
     // rows (cf_crs_build, when it fits): the entries again (padding to 4 per
     // row), chunk offsets and the split launches' range sums
-    if (r.kind == CF_FCI && !(da >= 400 && db <= cf::kEllMaxDb) && n >= 8192)
-        crs += n * (row + 3) * bytes_nnz + (n / 64 + 2) * 8 + (uint64_t)cf::kSellMaxSplit * n * 8;
-    const uint64_t krylov = (uint64_t)(ncv + 3) * n * 8;
-    return crs + krylov + ints + (64ull << 20);
+    const bool ell = da >= 400 && db <= cf::kEllMaxDb;
+    uint64_t solve = (uint64_t)(ncv + 3) * n * 8;  // Krylov basis
+    if (r.kind == CF_FCI && !ell && n >= 8192)
+        solve += n * (row + 3) * bytes_nnz + (n / 64 + 2) * 8 + (uint64_t)cf::kSellMaxSplit * n * 8;
+    // beside the CRS while it is built and before these: the rows' values (2 GiB or
+    // one alpha string's at a time) and the beta tables they are evaluated from
+    uint64_t build = 0;
+    if (r.kind == CF_FCI && db <= 65535) {
+        const uint64_t sb = (uint64_t)r.ndown * (L - r.ndown);
+        const uint64_t ddb = cf::binom_host(r.ndown, 2) * cf::binom_host(L - r.ndown, 2);
+        build = (1 + sb) * db * 4 + (1 + sb + ddb) * db * 12;
+        if (!ell) build += std::min(n * row * 8, std::max<uint64_t>(2ull << 30, row * db * 8));
+    }
+    return crs + std::max(solve, build) + ints + (64ull << 20);
 }
 
 void publish(cf_server* S, const cf_result& res, uint64_t footprint) {

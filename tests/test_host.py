@@ -136,6 +136,23 @@ def test_request_footprint_and_argument_checks():
         fp(CA.CF_FCI, 8, 9, 4)
 
 
+def test_request_footprint_covers_the_scratch_of_its_route():
+    def small_doci(npair):
+        h, V = np.zeros((16, 16)), np.zeros((16,) * 4)
+        r, _keep = CA.SolveServer._request(0, CA.CF_DOCI, h, V, npair, npair, None, 0.0, CA.CF_F64, 0, 0.0, 0, 0.0,
+                                           False, CA.CF_SOLVER_AUTO)
+        b = CA.C.c_uint64()
+        CA._check(CA.lib().cf_request_footprint(CA.C.byref(r), CA.C.byref(b)))
+        return b.value
+
+    # lock-step batch: diagonal, two images and three Krylov vectors a determinant (12,870 and 120 rows)
+    assert small_doci(8) - small_doci(2) >= 6 * 8 * (12870 - 120)
+    # stored FCI of L=16 0a6b (8,008 rows of 736 entries): CRS, and while it is built the rows'
+    # values and the beta tables (736 and 61 entries a string)
+    n, row, single = 8008, 736, 61
+    assert CA.SolveServer.footprint(CA.CF_FCI, 16, 0, 6, CA.CF_F64) >= n * row * (12 + 8 + 12) + n * single * 4
+
+
 def test_determinant_file_parser_matches_oracle(tmp_path):
     """Permutator_File::read_file semantics: '#' lines are comments, strings are
     binary with the highest orbital first, CR line ends are tolerated, lines
