@@ -1,5 +1,5 @@
-"""GPU tests of cf_solve_doci_batch: many small DOCI solves in one launch,
-one workgroup per request (the loop the reference runs one solve at a time:
+"""GPU tests of cf_solve_doci_batch: many small DOCI solves in lock step,
+one launch a Lanczos step (the loop the reference runs one solve at a time:
 OrbitalOptimization::update_cim -> set_ham -> build_ci -> solve,
 SimulatedAnnealing.cpp:83-87; DOCI::construct_CI_matrix, CIMethod.cpp:611-660).
 

@@ -1,7 +1,8 @@
-"""GPU tests of cf_solve_doci_batch at the edges of its workgroup shapes and
-splits: spaces of 2 to 13,312 rows around the three shapes' bounds, more
-requests than fill the GPU, tight tolerances (many steps) and a step limit
-that ends a solve, each against dense eigenvalues or the stored-matrix solve."""
+"""GPU tests of cf_solve_doci_batch over its workgroup shapes and splits: spaces
+of 2 to 12,870 rows, on either side of the shapes' bounds (1,001 and 1,140 rows;
+4,060 and 4,495), more requests than fill the GPU and than a grid dimension, and
+requests that stop early, late and at the step limit, against dense eigenvalues
+or the stored-matrix solve; the residual estimate against Lanczos in numpy."""
 import numpy as np
 import pytest
 
@@ -29,7 +30,7 @@ def stored_energy(q):
 
 
 @pytest.mark.parametrize("L,npair", [(2, 1), (4, 2), (8, 4), (12, 6), (14, 4), (13, 8), (14, 7), (15, 6), (16, 8),
-                                     (32, 1), (28, 2)])
+                                     (32, 1), (28, 2), (20, 3), (30, 3), (31, 3), (25, 4)])
 def test_batch_sizes(L, npair):
     q = request(L, npair, 40 + L + npair)
     res = CA.solve_doci_batch([dict(q), dict(q, tol=1e-9), dict(q, tol_energy=1e-9)])

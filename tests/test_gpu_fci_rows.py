@@ -2,7 +2,8 @@
 bit for bit against the oracle at the edges of the tiles (64 strings, 64
 positions) and of the chunks (512 strings), with elements that are dropped,
 after new integrals, in FP32 copies; and a space whose values take several
-passes (more than 2 GiB), against the on-the-fly product."""
+passes (more than 2 GiB), against the on-the-fly product; and the rows of a beta
+space above 65,535 strings, which are evaluated one by one."""
 from math import comb
 
 import numpy as np
@@ -60,3 +61,20 @@ def test_values_in_several_passes():
     row, col, val = cim.get_mat().export_upper(r0, n)
     ref = O.build_crs("FCI", h, V, na, nb, start=219, end=220)
     assert np.array_equal(row, ref.row) and np.array_equal(col, ref.col) and np.array_equal(val, ref.data)
+
+
+def test_rows_of_a_large_beta_space():
+    """77,520 strings of seven electrons: as beta strings (32-bit targets, one evaluation an
+    element and pass) and as alpha strings they are the same matrix, bit for bit."""
+    L, ne = 20, 7
+    h, V = CA.gen_integrals(L, 6)
+    beta, alpha = (CA.FCI(CA.Hamiltonian(h, V, *n)) for n in ((0, ne), (ne, 0)))
+    n, nnz, upper = beta.get_mat().info()
+    row = 1 + ne * (L - ne) + comb(ne, 2) * comb(L - ne, 2)
+    assert (n, nnz, upper) == (77520, 77520 * row, 77520 * (row + 1) // 2) == tuple(alpha.get_mat().info())
+    for r0 in (0, 31000, n - 500):
+        a, b = (m.get_mat().export_upper(r0, r0 + 500) for m in (alpha, beta))
+        assert all(np.array_equal(x, y) for x, y in zip(a, b))
+    x = np.random.default_rng(3).standard_normal(n)
+    y, z = beta.get_mat().mvprod(x), alpha.get_mat().mvprod(x)
+    assert np.linalg.norm(y - z) <= 1e-14 * np.linalg.norm(z)

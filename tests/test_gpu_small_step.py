@@ -1,8 +1,9 @@
-"""GPU tests of the two-launch Lanczos step of small spaces: energies, vectors
-and products against dense eigenvalues at the edges of its thread counts (n
-below a wavefront, of one, 1,024, 2,048, 5,120, 16,384 and above, where the
-other step takes over), across restarts, and through a breakdown (a start
-vector in a small invariant space)."""
+"""GPU tests of the two-launch Lanczos step of small spaces on each of its
+instances (up to 1,024, 2,048, 5,120, 10,240 and 16,384 rows, fewer than a
+wavefront included): energies and vectors against dense eigenvalues, or energies
+against the Davidson solve (also above 16,384 rows, where the other step takes
+over), across restarts, and through a breakdown (a start vector in a small
+invariant space)."""
 import numpy as np
 import pytest
 
@@ -19,7 +20,7 @@ def dense(m, n):
     return A
 
 
-# FCI dimensions 9, 36, 60, 400, 1000, 1225; DOCI 1716, 3432
+# FCI dimensions 9, 36, 50, 400, 100, 1225; DOCI 1716, 3432
 @pytest.mark.parametrize("kind,L,na,nb", [("FCI", 3, 1, 2), ("FCI", 4, 2, 2), ("FCI", 5, 2, 4), ("FCI", 6, 3, 3),
                                           ("FCI", 5, 2, 2), ("FCI", 7, 3, 4), ("DOCI", 13, 6, 6), ("DOCI", 14, 7, 7)])
 @pytest.mark.parametrize("ncv", [42, 12])
@@ -35,8 +36,8 @@ def test_against_dense(kind, L, na, nb, ncv):
     assert abs(x @ x - 1.0) <= 1e-12
 
 
-# 15,876 (in range), 19,404 (above)
-@pytest.mark.parametrize("L,na,nb", [(9, 4, 4), (10, 4, 3)])
+# 7,056, 10,584, 15,876 (in range), 25,200 (above)
+@pytest.mark.parametrize("L,na,nb", [(9, 3, 3), (9, 4, 3), (9, 4, 4), (10, 4, 3)])
 def test_around_the_bound(L, na, nb):
     h, V = CA.gen_integrals(L, 5)
     ci = CA.FCI(CA.Hamiltonian(h, V, na, nb))
