@@ -29,8 +29,8 @@
 // and np nv dependent-free gathers a row.  One workgroup per request, with the
 // test on one of its waves, left most CUs idle and waited for a column from L2
 // at every hop: 48 requests of L=14 (3,432 rows) took 9.1 ms on 48 of 256 CUs;
-// now a step is 13 us, a step with a test 20-30 us, and the batch 1.7 ms (a
-// whole call 10.9 -> 3.1 ms, the rest of it the integrals' way to the GPU).
+// now a step is 14.5 us on average, its test beside it, and the batch 1.4 ms (a
+// whole call 10.9 -> 2.7 ms, the rest of it the integrals' way to the GPU).
 #include "batch.h"
 
 #include <algorithm>

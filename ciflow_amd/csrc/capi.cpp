@@ -595,7 +595,7 @@ void build_crs_arrays(cf_crs* m) {
             largs.sidx = sidx.p;
             largs.L = H->L;
             KTimer t(c, "crs_count");
-            tables = make_det_tables(dtabs, sp->n, sp->dup.p, sp->ddown.p, skey.p, sidx.p, H->dev(), c->stream);
+            tables = make_det_tables(dtabs, sp->n, sp->dup.p, sp->ddown.p, skey.p, H->dev(), c->stream);
             if (tables) launch_det_rows_tab(dtabs, targs, false, c->stream);
             else launch_det_rows_lookup(largs, false, c->stream);
         } else {

@@ -121,8 +121,9 @@ __global__ void __launch_bounds__(256) k_bd_rotate(BdView b) {
 // to 24 basis vectors in registers (kChunk at a time, C chunks; rows past k
 // repeat row k - 1 with coefficient 0), forms t there and at once the dot
 // products V^T t that the next Gram-Schmidt pass needs.  HBM- and L2-bound: with
-// a pass of its own over V for those dots the vector passes of a step took 242 us
-// for 12 x FCI L=11 (5,5) and 123 us for 12 x DOCI L=19, now 167 and 85.
+// a pass of its own over V for those dots the vector passes of a step (the new
+// column's dots and the scaling included, mean over a solve) took 271 us for 12 x
+// FCI L=11 (5,5) and 131 us for 12 x DOCI L=19, now 192 and 95.
 // Workgroups of 512, at most 64 a lane: 183 VGPRs hold the 24-vector instance
 // (at the 128 of twice as many wavefronts it spilled 104).
 // The rows' addresses stay in scalar registers: a uniform base per row and a

@@ -35,12 +35,12 @@ struct DetTables {
 };
 
 // Builds the tables of a list of n distinct determinants from its sorted keys
-// (up << 32 | down) and their list indices.  False, with nothing built, for a
+// (up << 32 | down).  False, with nothing built, for a
 // list that they do not suit: repeated determinants, more than 16,384 strings
 // of a spin, or fewer than one determinant per 32 pairs of its strings (8 for
 // lists of fewer than 4,096), which also bounds pos to 32 entries each.
-bool make_det_tables(DetTables& T, uint64_t n, const str_t* up, const str_t* down, const uint64_t* skey,
-                     const uint32_t* sidx, HamDev H, hipStream_t stream);
+bool make_det_tables(DetTables& T, uint64_t n, const str_t* up, const str_t* down, const uint64_t* skey, HamDev H,
+                     hipStream_t stream);
 // Count pass (r.rowcnt) or fill pass (r.rowptr, col, val, val32) of the rows.
 // The fill writes a row's entries in the order of the sorted determinants:
 // ascending columns for a list in (up, down) order.

@@ -19,7 +19,7 @@
 //
 // What bounds it: two dependent loads from L2 (connection, pos) per candidate
 // and one for the element.  95,040 determinants of L=12 6a5b (120 alpha strings
-// times every beta string; 4.2e7 stored of 1.1e8 candidates): 4.7 ms per pass by
+// times every beta string; all of the 9.2e7 candidates are stored): 4.7 ms per pass by
 // lookup and 2.6 ms for the sort, now 0.78 (count) + 0.92 ms (fill); build, sliced
 // copy and first product 15.0 -> 3.25 ms.  Random lists: 95,000 of L=13 6.9 ->
 // 4.7 ms, 30,000 of L=10 4.1 -> 1.6 ms.  The tables' launches cost 0.1 ms, which
@@ -312,10 +312,9 @@ void connect(DetStrings& S, HamDev H, hipStream_t st) {
 
 }  // namespace
 
-bool make_det_tables(DetTables& T, uint64_t n, const str_t* up, const str_t* down, const uint64_t* skey,
-                     const uint32_t* sidx, HamDev H, hipStream_t st) {
+bool make_det_tables(DetTables& T, uint64_t n, const str_t* up, const str_t* down, const uint64_t* skey, HamDev H,
+                     hipStream_t st) {
     constexpr uint64_t kMost = 16384;
-    (void)sidx;
     if (!n || n > 0x7fffffffull) return false;
     DBuf<unsigned int> dup(1);
     k_fill_u32<<<1, 256, 0, st>>>(1, 0u, dup.p);

@@ -321,7 +321,9 @@ void launch_finish_step_r(uint64_t n, int j, const double* c1, const double* c2,
 // launches, now 19 (6.1 + 4.3 us and 8.9 for the product); DOCI L=10 (252) 23 ->
 // 10 us.  An optimisation step of the two: 4.8 -> 2.85 and 2.07 -> 1.19 ms.  From
 // 16,384 rows on the vector read by every workgroup would cost more than the
-// launches saved.
+// launches saved.  (Above 10,240 rows k_step_dots holds 64 doubles a thread and
+// spills 42 of its 128 VGPRs; a product and its step still take 53 us instead of
+// 63 for FCI L=9 (15,876 rows) and 32 instead of 41 for DOCI L=16 (12,870).)
 // ---------------------------------------------------------------------------
 template <int R>
 __global__ void __launch_bounds__(1024) k_step_dots(int n, int j, const double* __restrict__ Vb,

@@ -424,7 +424,7 @@ extern "C" {
 // CF_PREC_AUTO: FP32 values only where the request's route stores matrix
 // values (a stored CRS); the small-DOCI batch, the lock-step Davidson
 // batch and the on-the-fly sigma read none, and FP64 is as fast or faster
-// there (measured per class on MI355X: FP64 lock-step batches 0-21% more
+// there (measured per class on MI355X: FP64 lock-step batches 6-30% more
 // solves/s, the FP32 phase ending in 3-12 extra FP64 polish products).
 static cf_request resolve_precision(const cf_request& r) {
     cf_request q = r;

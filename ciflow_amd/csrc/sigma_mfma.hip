@@ -20,9 +20,11 @@
 // (L=11: 66 = 4 * 16 + 2).
 //
 // Bound by the MFMAs: 2 * 16 ceil(d_b / 16) * 4 ceil(|A| / 4) * 16 tiles flop per Ia.
-// L=12 (6,6), d = 853,776: 183 us, whole sigma 243 us (433 with ab3's pair by
-// pair actions); 12 vectors of L=11 (5,5), d = 213,444: 256 us (468).  The
-// MFMAs alone are 77 and 158 us at the card's 69.4 TFLOP/s.
+// L=12 (6,6), d = 853,776: 188 us, whole sigma 243 us (433 with ab3's pair by
+// pair actions); 12 vectors of L=11 (5,5), d = 213,444: 353 us (627).  The
+// MFMAs alone are 79 and 151 us at the card's 69.4 TFLOP/s, the rest the gathers
+// and the barriers around them.  Two of the instances are at the limit of their
+// registers: <8, 4> (L=11) spills 4 of 128 VGPRs, <10, 8> (L=12) 8 of 256.
 #include "sigma.h"
 
 #include <algorithm>
@@ -71,8 +73,8 @@ MfmaShape shape_of(const SigmaArgs& a) {
 // fours, the rest pointing at a row of zeros -- so that several codes and LDS
 // reads are in flight at once.  k_mfma_count finds the longest lists (at most
 // 16: a string has one action per pair), k_mfma_gather fills.  (Codes of 16
-// bits, all of a tile's loaded before the barrier, spilled: 259 and 204 us
-// instead of 256 and 183.)
+// bits, all of a tile's loaded before the barrier, spilled more: 204 us instead of
+// 183 at L=12, and no gain at L=11.)
 template <class Put>
 __device__ __forceinline__ void beta_actions(const Exc* l, int Sb, uint32_t Ib, str_t bits, Put&& put) {
     for (int e = 0; e < Sb; ++e)

@@ -242,7 +242,7 @@ struct BlockSums {
 // reads and ten VALU operations a hop, and was latency-bound.  A wavefront without
 // rows of the block only stages.  L=23 (11 pairs), n = 1,352,078: 95 -> 81 us; 12
 // vectors of L=19 (9 pairs), n = 92,378: 71 -> 46 us.  What is left: LDS and VALU
-// are busy 45% and 40% of the time, the rest is waits (a workgroup's stages follow
+// are busy 45% and 43% of the time, the rest is waits (a workgroup's stages follow
 // each other); blocks sorted by c, 512 threads of one row (90 us) and the table
 // words loaded ahead (83) did not help.
 struct DociInst {
